@@ -35,6 +35,8 @@ namespace ssids_hip {
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef double double16_t __attribute__((ext_vector_type(16)));
+typedef unsigned uint16v_t __attribute__((ext_vector_type(16)));
 
 // front of workgroup b in a level table, or -1 past the table's total (grids
 // sized for the plan's capacities may be larger than the level needs)
@@ -60,20 +62,27 @@ __device__ inline const double *child_src(const NodeDev &c, int kr, int k) {
 }
 
 // ---------------------------------------------------------------------------
-// Diagonal block factorization, NW waves per front.  Lane j of wave v keeps
-// rows [vR, vR+R) (R = 64/NW) of column j of the symmetric w x w block in
+// Diagonal block factorization, NW waves per front.  Lane i of wave v keeps
+// columns [vR, vR+R) (R = 64/NW) of row i of the symmetric w x w block in
 // registers; pivots are tracked in a uniform bit mask (no physical swaps).
-// Per pivot step:
-//  * search: every lane scans its live rows i >= j for max |a(i,j)| (the
-//    lower triangle, as block_ldlt.hxx:77-101 searches it: each symmetric
-//    pair once, in one orientation, so a maximum off the diagonal gives the
-//    pair (column, row) with column < row whatever the rounding of the two
-//    mirrored entries; rows ascending, first maximum kept); each wave
-//    reduces to its (value, smallest column, that column's row) with DPP
-//    and a ballot, and the waves' candidates are merged through LDS in the
-//    same order;
-//  * the owners of the pivot column(s) broadcast them through LDS;
-//  * rank-1 / rank-2 update of every column's rows in registers;
+// Per pivot step, with one workgroup barrier unless the maximum lies off the
+// diagonal:
+//  * search: every lane takes the maximum |a(i,j)| of its live columns j <= i
+//    (the lower triangle, as block_ldlt.hxx:77-101 searches it: each
+//    symmetric pair once, in one orientation, so a maximum off the diagonal
+//    gives the pair (column, row) with column < row whatever the rounding of
+//    the two mirrored entries).  The wave reduces the maxima's high words
+//    with DPP; the low words, and the order (smallest column, then row) among
+//    equal values, are looked at only when two lanes share the high word;
+//  * each wave publishes its candidate through LDS before the barrier: the
+//    value, its position, its reciprocal (the division runs while the
+//    position is found) and the whole column, which one wave holds, so no
+//    second exchange follows the merge.  The waves hold ascending columns,
+//    so the first wave with the largest value has the smallest column;
+//  * a maximum off the diagonal fetches the second column the same way;
+//  * rank-1 / rank-2 update of every row's columns in registers: the lane's
+//    own column entry times L of the wave's R columns, which sit in the lanes
+//    of each row of 16 and reach the FMAs by DPP (row_newbcast);
 //  * the L column(s) of the step go to LDS, indexed by elimination step.
 // Pivot rules of src/ssids/cpu/kernels/block_ldlt.hxx:289-414: maximum on the
 // diagonal -> 1x1; else the 2x2 test of block_ldlt.hxx:213-218, else the
@@ -81,8 +90,214 @@ __device__ inline const double *child_src(const NodeDev &c, int kr, int k) {
 // index a zero pivot.  The a posteriori test of k_apply then checks
 // |l| <= 1/u over the full column.  The elimination order lp[] permutes the
 // block on write back.
+// The block is bound by the chain of its 64 steps on one CU: about 300
+// instructions of one wave per SIMD at 4 cycles, two LDS round trips and a
+// barrier (1,760 cycles a step, 132,000 a block).  The layout with a column
+// per lane and 16 rows a wave needed the search's merge and the column's
+// broadcast one after the other, two barriers a step: 250,000 cycles, 118 us
+// a block against 64 us (64 x 64, one front).  Eight waves of 8 columns take
+// 83 us: the second wave of a SIMD waits for its issue slots.
 // ---------------------------------------------------------------------------
 constexpr int kDiagWaves = 4;
+constexpr int kDiagCols = kBlk / kDiagWaves;  // columns of a wave: 16
+
+// max of two values that hold no signalling NaN (a NaN loses), one
+// instruction: fmax would quiet both operands first
+__device__ inline double max_f64(double x, double y) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+// a condition every lane of the wave agrees on, as a scalar
+__device__ inline bool uniform_true(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0ull; }
+
+// v permuted within rows of lanes by a DPP control
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+  const int hi = __double2hiint(v), lo = __double2loint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, true));
+}
+// the larger of v and its permuted value (no NaN)
+template <int CTRL>
+__device__ inline double dpp_max_f64(double v) {
+  const double o = dpp_f64<CTRL>(v);
+  return o > v ? o : v;
+}
+
+// value of v in lane j (j uniform), as a scalar
+__device__ inline double lane_value(double v, int j) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
+                          __builtin_amdgcn_readlane(__double2loint(v), j));
+}
+
+// Largest |a[j]| over j = 0..15 in the lanes >= c0 + j only (the lower
+// triangle of a wave's columns); NaN never wins.  Called with every lane of
+// the wave active.
+__device__ __forceinline__ double max_lower(double16_t a, int c0) {
+  double m0 = 0.0, m1 = 0.0;
+#define SSIDS_MAX(m, r) \
+  "v_max_f64 %" #m ", %" #m ", |%" #r "|\n\ts_lshl_b64 exec, exec, 1\n\t"
+  asm("s_lshl_b64 exec, -1, %18\n\t" SSIDS_MAX(0, 2) SSIDS_MAX(1, 3) SSIDS_MAX(0, 4)
+          SSIDS_MAX(1, 5) SSIDS_MAX(0, 6) SSIDS_MAX(1, 7) SSIDS_MAX(0, 8) SSIDS_MAX(1, 9)
+              SSIDS_MAX(0, 10) SSIDS_MAX(1, 11) SSIDS_MAX(0, 12) SSIDS_MAX(1, 13)
+                  SSIDS_MAX(0, 14) SSIDS_MAX(1, 15) SSIDS_MAX(0, 16) SSIDS_MAX(1, 17)
+      "s_mov_b64 exec, -1"
+      : "+v"(m0), "+v"(m1)
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]),
+        "v"(a[7]), "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]),
+        "v"(a[14]), "v"(a[15]), "s"(c0)
+      : "scc");
+#undef SSIDS_MAX
+  return max_f64(m0, m1);
+}
+
+// One bit per j: h[j] = m in this lane (bit 15 - j).  The compares go to four
+// scalar pairs in turn, so that no add-with-carry waits for the compare just
+// before it.
+__device__ __forceinline__ unsigned equal_bits(uint16v_t h, unsigned m) {
+  unsigned bits = 0;
+  unsigned long long s0, s1, s2, s3;
+#define SSIDS_EQ4(j)                                                                   \
+  asm("v_cmp_eq_u32 %1, %5, %9\n\tv_cmp_eq_u32 %2, %6, %9\n\t"                         \
+      "v_cmp_eq_u32 %3, %7, %9\n\tv_cmp_eq_u32 %4, %8, %9\n\t"                         \
+      "v_addc_co_u32 %0, vcc, %0, %0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, %2\n\t"     \
+      "v_addc_co_u32 %0, vcc, %0, %0, %3\n\tv_addc_co_u32 %0, vcc, %0, %0, %4"         \
+      : "+v"(bits), "=&s"(s0), "=&s"(s1), "=&s"(s2), "=&s"(s3)                         \
+      : "v"(h[j]), "v"(h[j + 1]), "v"(h[j + 2]), "v"(h[j + 3]), "s"(m)                 \
+      : "vcc")
+  SSIDS_EQ4(0);
+  SSIDS_EQ4(4);
+  SSIDS_EQ4(8);
+  SSIDS_EQ4(12);
+#undef SSIDS_EQ4
+  return bits;
+}
+
+// a[j] = fma(c, l_j, a[j]) for j = 0..15, l_j the value of `l` in lane j of
+// the lane's own row of 16; with `two`, a[j] = fma(c2, l2_j, a[j]) first.
+// The leading s_nop separates the writes of l and l2 from their DPP reads.
+// The branch sits inside the statement, so that the registers stay where
+// they are on both paths.
+__device__ __forceinline__ void rank_update(double16_t &a, double c, double l, int two,
+                                            double c2, double l2) {
+#define SSIDS_FMAC(n, l, c) \
+  "v_fmac_f64_dpp %" #n ", %" #l ", %" #c " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
+#define SSIDS_FMAC16(l, c)                                                               \
+  SSIDS_FMAC(0, l, c) SSIDS_FMAC(1, l, c) SSIDS_FMAC(2, l, c) SSIDS_FMAC(3, l, c)         \
+  SSIDS_FMAC(4, l, c) SSIDS_FMAC(5, l, c) SSIDS_FMAC(6, l, c) SSIDS_FMAC(7, l, c)         \
+  SSIDS_FMAC(8, l, c) SSIDS_FMAC(9, l, c) SSIDS_FMAC(10, l, c) SSIDS_FMAC(11, l, c)       \
+  SSIDS_FMAC(12, l, c) SSIDS_FMAC(13, l, c) SSIDS_FMAC(14, l, c) SSIDS_FMAC(15, l, c)
+  double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], a4 = a[4], a5 = a[5], a6 = a[6],
+         a7 = a[7], a8 = a[8], a9 = a[9], a10 = a[10], a11 = a[11], a12 = a[12], a13 = a[13],
+         a14 = a[14], a15 = a[15];
+  asm("s_nop 1\n\ts_cmp_eq_u32 %20, 0\n\ts_cbranch_scc1 .Lrank1_%=\n\t" SSIDS_FMAC16(18, 19)
+      ".Lrank1_%=:\n\t" SSIDS_FMAC16(16, 17)
+      : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7),
+        "+v"(a8), "+v"(a9), "+v"(a10), "+v"(a11), "+v"(a12), "+v"(a13), "+v"(a14), "+v"(a15)
+      : "v"(l), "v"(c), "v"(l2), "v"(c2), "s"(two)
+      : "scc");
+  a[0] = a0, a[1] = a1, a[2] = a2, a[3] = a3, a[4] = a4, a[5] = a5, a[6] = a6, a[7] = a7;
+  a[8] = a8, a[9] = a9, a[10] = a10, a[11] = a11, a[12] = a12, a[13] = a13, a[14] = a14,
+  a[15] = a15;
+#undef SSIDS_FMAC16
+#undef SSIDS_FMAC
+}
+
+// Rows 16b..16b+15 of the inverse's diagonal block b: lane j of every row of
+// 16 lanes holds column j in m, and lane i of a row holds L(i, k) in lk[k];
+// m[i] -= L(i, k) m[k] for k ascending, L by DPP.
+template <int K>
+__device__ __forceinline__ void unit_lower_columns(double (&m)[16], const double (&lk)[15]) {
+  if constexpr (K < 15) {
+    const double c = -m[K];
+#pragma unroll
+    for (int i = K + 1; i < 16; ++i)
+      asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+          : "+v"(m[i])
+          : "v"(lk[K]), "v"(c), "n"(i));
+    unit_lower_columns<K + 1>(m, lk);
+  }
+}
+
+// W (64 x 64 row-major) = M = (I + N)^{-1}, N the strictly lower matrix with
+// N(i, k) = mi[k][i]; ms is scratch.  Wave b inverts the 16 x 16 diagonal
+// block b in registers, then blocks join by pairs on FP64 MFMA:
+//   [M11 0; -M22 (L21 M11) M22]
+// first to 32 x 32 (two waves), then to 64 x 64 (a 16 x 16 tile a wave).  A
+// product's result (row i, column j in lane j + 16 (i % 4), register i / 4)
+// is the next product's right operand as it stands.  Against 63 substitution
+// steps on all 64 rows (7.5 us a block, most of it instruction fetch of the
+// unrolled steps) this takes about 1 us.
+__device__ __forceinline__ void block_inverse(const double (&mi)[kBlk][kBlk + 1],
+                                              double (&ms)[kBlk][kBlk + 1], int wv, int lane,
+                                              gdouble *W) {
+  const int ri = lane & 15, kq = lane >> 4;
+  {
+    const int b0 = 16 * wv;
+    double lk[15], m[16];
+#pragma unroll
+    for (int k = 0; k < 15; ++k) lk[k] = mi[b0 + k][b0 + ri];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m[i] = (i == ri) ? 1.0 : 0.0;
+    // the loads above have returned and their last reader below is two
+    // instructions away from any write of a DPP source
+    asm volatile("s_nop 1");
+    unit_lower_columns<0>(m, lk);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if ((i >> 2) == kq) ms[b0 + i][b0 + ri] = m[i];
+  }
+  __syncthreads();
+  // acc += A B over 16 pivots, A(i, k) from `ld`, B(k, j) in b[k / 4]
+  auto mul = [&](double4_t &acc, const double (&A)[kBlk][kBlk + 1], int r, int c, bool trans,
+                 const double4_t &b) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const double av = trans ? A[c + 4 * u + kq][r + ri] : A[r + ri][c + 4 * u + kq];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b[u], acc, 0, 0, 0);
+    }
+  };
+  auto right = [&](int r, int c) {  // the block of M at (r, c) as a right operand
+    double4_t b;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) b[u] = ms[r + 4 * u + kq][c + ri];
+    return b;
+  };
+  auto put = [&](int r, int c, const double4_t &v) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) ms[r + 4 * u + kq][c + ri] = -v[u];
+  };
+  const double4_t zero = {0.0, 0.0, 0.0, 0.0};
+  if (wv < 2) {
+    const int b0 = 32 * wv;
+    double4_t x = zero, y = zero;
+    mul(x, mi, b0 + 16, b0, true, right(b0, b0));
+    mul(y, ms, b0 + 16, b0 + 16, false, x);
+    put(b0 + 16, b0, y);
+  }
+  __syncthreads();
+  {
+    // tile (I, J) of the lower left 32 x 32; X = L21 M11 for column block J
+    const int I = wv >> 1, J = wv & 1;
+    double4_t x0 = zero, x1 = zero, y = zero;
+    for (int k = J; k < 2; ++k) {  // M11 is lower triangular by blocks
+      const double4_t b = right(16 * k, 16 * J);
+      mul(x0, mi, 32, 16 * k, true, b);
+      mul(x1, mi, 48, 16 * k, true, b);
+    }
+    mul(y, ms, 32 + 16 * I, 32, false, x0);
+    if (I == 1) mul(y, ms, 48, 48, false, x1);
+    put(32 + 16 * I, 16 * J, y);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < 16; ++it) {
+    const int r = 16 * wv + it;
+    W[r * kBlk + lane] = masked(ms[r][lane], (lane >> 4) <= wv);
+  }
+}
 
 constexpr int kGT = 64;  // gather tile edge
 
@@ -115,13 +330,19 @@ template <int NW, bool FIRST, bool C32>
 __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl_slots,
                                                   int step, FactorParams fp, GatherArgs ga) {
   constexpr int R = kBlk / NW;
+  static_assert(NW == kDiagWaves && R == kDiagCols, "a row of lanes holds L of a wave's columns");
   __shared__ double t[kBlk][kBlk + 1];  // load staging, then L by step: t[k][row]
-  __shared__ double cs2[2][2][kBlk];    // broadcast pivot columns (by step parity)
-  __shared__ unsigned long long ckey[2][NW];
-  __shared__ int ccr[2][NW];  // candidate column << 7 | row
+  __shared__ double ccol[2][NW][kBlk];  // the waves' candidate columns (by step parity)
+  struct alignas(16) Cand {
+    int lo, hi;  // |value|
+    int code;    // column << 6 | row
+    int pad;
+  };
+  __shared__ Cand cand[2][NW];
+  __shared__ double col2[kBlk];                // column of an off-diagonal maximum's row
   __shared__ double dinv[2 * kBlk + 2];
   __shared__ int lp[kBlk], inv_lp[kBlk], kind[kBlk];
-  __shared__ double mi[kBlk][kBlk + 1];  // inverse of L_bb (elimination order)
+  __shared__ double mi[kBlk][kBlk + 1];  // L_bb's strict lower part by columns
   int s;
   if constexpr (FIRST) {
     static_assert(64 * NW == kThreads, "one workgroup shape for both phases");
@@ -137,7 +358,7 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
   }
   NodeDev &N = nodes[s];
   if (step >= N.nsteps) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r0 = wv * R;
+  const int tid = threadIdx.x, lane = tid & 63, wv = uni((int)threadIdx.x >> 6), c0 = wv * R;
   int p, q;
   if (step == 0) {
     p = 0;
@@ -157,248 +378,264 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
   if (w == 0) return;
   const int ldl = N.ldl;
   double *L = N.L;
-  {
-    // the w x w block (lower triangle mirrored), zero outside; every thread's
-    // loads are unconditional (indices clamped into the block) so they are
-    // all in flight together
+  // The block's lower triangle, t[row][column] (a front's first block is still
+  // there from its assembly); every thread's loads are unconditional (indices
+  // clamped into the block) so they are all in flight together.
+  if constexpr (!FIRST) {
     gcdouble *Lg = (gcdouble *)L;
-    gdouble *dbak = (gdouble *)N.dbak;
-    double v[kBlk * kBlk / (64 * NW)];
+    double v[R];
 #pragma unroll
-    for (int it = 0; it < kBlk * kBlk / (64 * NW); ++it) {
-      const int idx = tid + it * 64 * NW, r = idx % kBlk, c = idx / kBlk;
-      v[it] = masked(Lg[(size_t)(p + imin(c, w - 1)) * ldl + p + imin(r, w - 1)],
-                     r >= c && r < w);
-    }
+    for (int j = 0; j < R; ++j)
+      v[j] = Lg[(size_t)(p + imin(c0 + j, w - 1)) * ldl + p + imin(lane, w - 1)];
 #pragma unroll
-    for (int it = 0; it < kBlk * kBlk / (64 * NW); ++it) {
-      const int idx = tid + it * 64 * NW, r = idx % kBlk, c = idx / kBlk;
-      if (r >= c) {
-        t[r][c] = v[it];
-        t[c][r] = v[it];
-        if (r < w) {
-          dbak[r + c * kBlk] = v[it];
-          dbak[c + r * kBlk] = v[it];
-        }
-      }
-    }
+    for (int j = 0; j < R; ++j) t[lane][c0 + j] = v[j];
   }
   if (tid < kBlk) N.colmax[tid] = 0ull;
   __syncthreads();
-  double a[R];
+  double16_t a;   // columns c0 .. c0 + 15 of row `lane`, zero outside the block
+  uint16v_t msk;  // high-word mask of the search (0 above the diagonal)
 #pragma unroll
-  for (int r = 0; r < R; ++r) a[r] = t[r0 + r][lane];
+  for (int j = 0; j < R; ++j) {
+    a[j] = masked(t[imax(lane, c0 + j)][imin(lane, c0 + j)], lane < w && c0 + j < w);
+    msk[j] = (lane >= c0 + j) ? 0x7fffffffu : 0u;
+  }
+  {
+    // the backup the failed columns are restored from, a column a store
+    gdouble *dbak = (gdouble *)N.dbak;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if (lane < w) dbak[lane + (c0 + j) * kBlk] = a[j];
+  }
   __syncthreads();
-  unsigned long long elim = (w < 64) ? (~0ull << w) : 0ull;  // eliminated / absent
-  int k = 0, par = 0;
-  // every remaining index becomes a zero pivot, in increasing index order;
-  // code -6: a non-positive pivot of the positive-definite factorization
-  auto zero_rest = [&](int code) {
-    int kk = k;
-    for (int i = 0; i < w; ++i) {
-      if ((elim >> i) & 1ull) continue;
-      if (wv == 0) t[kk][lane] = 0.0;
-      if (tid == 0) {
-        lp[kk] = i;
-        kind[kk] = 0;
-        dinv[2 * kk] = 0.0;
-        dinv[2 * kk + 1] = 0.0;
+  int livem = (lane < w) ? -1 : 0;  // -1: row `lane` is not eliminated
+  int k = 0, par = 0, stop = 0;
+  // a maximum below `small`, or of exactly zero, ends the block
+  const double small = !(fp.small <= 4.9406564584124654e-324) ? fp.small
+                                                              : 4.9406564584124654e-324;
+  const int sl = c0 + (lane & (R - 1));  // the column whose L this lane passes to rank_update
+  int plp = 0;  // lane k: pivot k's index | kind << 8 and D^{-1} entries
+  double pd0 = 0.0, pd1 = 0.0;
+  // v in the live rows, zero elsewhere
+  auto live_value = [&](double v) {
+    return __hiloint2double(__double2hiint(v) & livem, __double2loint(v) & livem);
+  };
+  // The end of a step: pivot pv's update a -= z (the lane's row) L (the wave's
+  // columns, ls of lane sl), after z2, ls2 of a 2x2 block's second column
+  // (two); L(:, k) = lj to LDS (every wave has the column: each stores its
+  // rows); D^{-1} to lane k.  The pivot's own column takes the coefficient 1
+  // and becomes exactly zero, out of the search; the published columns hold
+  // zeros for eliminated rows, so it stays zero.
+  auto finish = [&](int pv, double z, double ls, double lj, double e0, double e1, int two,
+                    double z2, double ls2) __attribute__((always_inline)) {
+    ls = (sl == pv) ? 1.0 : ls;
+    rank_update(a, -z, ls, two, -z2, ls2);
+    if (lane / R == wv) t[k][lane] = lj;
+    const bool mine = lane == k;
+    plp = mine ? (pv | (two + 1) << 8) : plp;
+    pd0 = mine ? e0 : pd0;
+    pd1 = mine ? e1 : pd1;
+    livem = (lane == pv) ? 0 : livem;
+    k += two + 1;
+  };
+  // The LDS exchanges alternate between two buffers: a wave that publishes
+  // the next step's candidate must not overwrite what a slower wave still
+  // reads of this one's.
+  if (fp.posdef) {
+    // Cholesky order: the lowest remaining index, always 1x1
+    do {
+      const double cv = a[k & (R - 1)];
+      if (wv == k / R) ccol[par][0][lane] = live_value(cv);
+      __syncthreads();
+      const double z = ccol[par][0][lane], zs = ccol[par][0][sl];
+      par ^= 1;
+      const double d = lane_value(z, k);
+      if (!uniform_true(d > 0.0)) {
+        stop = -6;
+        break;
       }
-      ++kk;
+      const double e0 = 1.0 / d;
+      finish(k, z, zs * e0, z * e0, e0, 0.0, 0, 0.0, 0.0);
+    } while (k < w);
+  } else {
+    do {
+      // ---- search this lane's live columns, by the high words
+      uint16v_t h;
+#pragma unroll
+      for (int j = 0; j < R; ++j) h[j] = (unsigned)__double2hiint(a[j]) & msk[j];
+      unsigned m0 = max(max(h[0], h[1]), h[2]), m1 = max(max(h[3], h[4]), h[5]);
+#pragma unroll
+      for (int j = 6; j < R - 2; j += 4) {
+        m0 = max(max(m0, h[j]), h[j + 1]);
+        m1 = max(max(m1, h[j + 2]), h[j + 3]);
+      }
+      m0 = max(max(m0, h[R - 2]), h[R - 1]);
+      const unsigned mh = max(m0, m1) & (unsigned)livem;
+      const unsigned H = (unsigned)uni((int)wave_max_u32(mh));
+      const unsigned long long hit = __builtin_amdgcn_ballot_w64(mh == H);
+      // the wave's candidate: row ci, column c0 + cj, |value| = (mhi, mlo)
+      int ci = __builtin_ctzll(hit);
+      const unsigned eq = (unsigned)__builtin_amdgcn_readlane((int)equal_bits(h, H), ci);
+      int cj;
+      unsigned mhi, mlo;
+      double cv;
+      if (__builtin_expect(
+              __builtin_popcountll(hit) + __builtin_popcount(eq) + (H >= 0x7ff00000u ? 1 : 0) == 2,
+              1)) {
+        cj = __builtin_clz(eq) - (32 - R);
+        cv = a[cj];
+        mhi = H;
+        mlo = (unsigned)__builtin_amdgcn_readlane(__double2loint(cv), ci);
+      } else {
+        // Two entries share the largest high word, or it is zero, a
+        // subnormal's or a NaN's.
+        unsigned low = 0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) low |= msk[j] ? (unsigned)__double2loint(a[j]) : 0u;
+        cj = ci = 0;
+        mhi = mlo = 0u;
+        // (zeros only: every column of the wave is eliminated)
+        if (H != 0u || uniform_true((low & (unsigned)livem) != 0u)) {
+          // exact maxima (NaN never wins), then the smallest column and row
+          const double mx = max_lower(a, c0);
+          const unsigned long long ml =
+              livem ? (unsigned long long)__double_as_longlong(mx) : 0ull;
+          const unsigned long long kw = wave_max_u64(ml);
+          int jf = R - 1;
+#pragma unroll
+          for (int j = R - 2; j >= 0; --j) jf = (fabs(a[j]) == mx) ? j : jf;
+          const unsigned code =
+              ~wave_max_u32((livem && ml == kw) ? ~(unsigned)((jf << 6) | lane) : 0u);
+          cj = uni((int)(code >> 6) & (R - 1));
+          ci = uni((int)(code & 63u));
+          mhi = (unsigned)uni((int)(kw >> 32));
+          mlo = (unsigned)uni((int)(kw & 0xffffffffull));
+        }
+        cv = a[cj];
+      }
+      ccol[par][wv][lane] = live_value(cv);
+      Cand c;
+      c.lo = (int)mlo;
+      c.hi = (int)mhi;
+      c.code = ((c0 + cj) << 6) | ci;
+      c.pad = 0;
+      if (lane == 0) cand[par][wv] = c;
+      __syncthreads();
+      // the first wave holding the largest value wins: lane u looks at wave
+      // u % NW's candidate
+      const Cand cu = cand[par][lane & (NW - 1)];
+      const double vm = __hiloint2double(cu.hi, cu.lo);
+      const double vmax = dpp_max_f64<0x4E>(dpp_max_f64<0xB1>(vm));
+      const int win = __builtin_ctzll(__builtin_amdgcn_ballot_w64(vm == vmax));
+      const double x0 = ccol[par][win][lane], y0 = ccol[par][win][sl];
+      par ^= 1;
+      const double rcp = 1.0 / vmax;  // in the shadow of the column's loads
+      const int code = __builtin_amdgcn_readlane(cu.code, win);
+      const int p1 = code >> 6, r1 = code & 63;
+      if (!uniform_true(vmax >= small)) {
+        stop = -5;
+        break;
+      }
+      const double a11 = lane_value(x0, p1);
+      int pv = p1, two = 0;
+      double z = x0, z2 = 0.0, ls2 = 0.0;
+      // 1 / a11 = the reciprocal of |a11| with the pivot's sign
+      double e0 = copysign(rcp, a11), e1 = 0.0;
+      double ls = y0 * e0;
+      if (__builtin_expect(p1 != r1, 0)) {
+        // ---- off the diagonal: column r1 as well
+        const double cv2 = a[r1 & (R - 1)];
+        if (wv == r1 / R) col2[lane] = live_value(cv2);
+        __syncthreads();
+        const double y = col2[lane], ys = col2[sl];
+        const double a21 = lane_value(x0, r1), a22 = lane_value(y, r1);
+        // explicit fma throughout the block (no contraction left to the
+        // compiler), so the oracle's restatement can round the same way;
+        // detscale = 1 / |a21| (the largest entry)
+        const double detscale = rcp;
+        const double detpiv = fma(a11 * detscale, a22, -fabs(a21));
+        if (uniform_true(fabs(detpiv) >= fabs(a21) / 2)) {
+          two = 1;
+          e0 = (a22 * detscale) / detpiv;
+          e1 = (-a21 * detscale) / detpiv;
+          const double e3 = (a11 * detscale) / detpiv;
+          const double l2 = fma(e1, x0, e3 * y), l2s = fma(e1, y0, e3 * ys);
+          if (lane / R == wv) t[k + 1][lane] = l2;
+          if (lane == k + 1) {
+            plp = r1 | 3 << 8;
+            pd0 = INFINITY;
+            pd1 = e3;
+          }
+          livem = (lane == r1) ? 0 : livem;
+          // column r1 becomes a - y 1 = 0 first and column p1 a - x 1 = 0 next
+          z2 = y;
+          ls2 = sl == r1 ? 1.0 : sl == p1 ? 0.0 : l2s;
+          ls = sl == r1 ? 0.0 : fma(e0, y0, e1 * ys);
+        } else {
+          // the larger diagonal as a 1x1 pivot
+          const bool first = uniform_true(fabs(a11) > fabs(a22));
+          e0 = 1.0 / (first ? a11 : a22);
+          pv = first ? p1 : r1;
+          z = first ? x0 : y;
+          ls = (first ? y0 : ys) * e0;
+        }
+      }
+      finish(pv, z, ls, fma(e0, z, e1 * z2), e0, e1, two, z2, ls2);
+    } while (k < w);
+  }
+  if (wv == 1) {
+    if (lane < k) {
+      lp[lane] = plp & 63;
+      kind[lane] = plp >> 8;
+      dinv[2 * lane] = pd0;
+      dinv[2 * lane + 1] = pd1;
     }
-    if (tid == 0) {
-      if (code == -6) {
+    // the rest: every remaining index a zero pivot, in increasing index
+    // order (stop -6: a non-positive pivot of the positive-definite
+    // factorization)
+    const unsigned long long rest = __builtin_amdgcn_ballot_w64(livem != 0);
+    if (stop != 0 && livem) {
+      const int kk = k + __popcll(rest & ((1ull << lane) - 1ull));
+      lp[kk] = lane;
+      kind[kk] = 0;
+      dinv[2 * kk] = 0.0;
+      dinv[2 * kk + 1] = 0.0;
+    }
+    if (stop != 0 && lane == 0) {
+      if (stop == -6) {
         N.flag = -6;
       } else {
         N.nzero += w - k;
         if (!fp.action) N.flag = -5;
       }
     }
-    k = w;
-  };
-  int cpar = 0;
-  while (k < w) {
-    // parity-buffered: a step with one barrier (positive definite) must not
-    // overwrite the columns a slower wave still reads from the step before
-    double (*cs)[kBlk] = cs2[cpar];
-    cpar ^= 1;
-    int bc, brow;
-    if (fp.posdef) {
-      // Cholesky order: the lowest remaining index, always 1x1
-      bc = brow = __ffsll((long long)~elim) - 1;
-    } else {
-      const bool live = !((elim >> lane) & 1ull);
-      // ---- search this lane's live rows
-      double bv = 0.0;
-      int br = 64;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {  // NaN never wins; all-zero keeps br = 64
-        const double av = fabs(a[r]);
-        const bool take = r0 + r >= lane && !((elim >> (r0 + r)) & 1ull) && av > bv;
-        bv = take ? av : bv;
-        br = take ? r0 + r : br;
-      }
-      // ---- wave candidate: value, then smallest column, then its row
-      const unsigned long long key = live ? (unsigned long long)__double_as_longlong(bv) : 0ull;
-      const unsigned long long kw = wave_max_u64(key);
-      const unsigned long long hit = __ballot(live && key == kw);
-      const int cw = hit ? __ffsll((long long)hit) - 1 : 64;
-      const int rw = hit ? __builtin_amdgcn_readlane(br, cw) : 64;
-      if (lane == 0) {
-        ckey[par][wv] = kw;
-        ccr[par][wv] = (cw << 7) | rw;
-      }
-      __syncthreads();
-      // largest value; among the waves holding it, smallest column, then row
-      unsigned long long kv[NW];
-      int cr[NW];
-#pragma unroll
-      for (int v = 0; v < NW; ++v) {
-        kv[v] = ckey[par][v];
-        cr[v] = ccr[par][v];
-      }
-      unsigned long long kmax = kv[0];
-#pragma unroll
-      for (int v = 1; v < NW; ++v) kmax = (kv[v] > kmax) ? kv[v] : kmax;
-      int best = 1 << 30;  // above every encoding; kmax is some wave's key
-#pragma unroll
-      for (int v = 0; v < NW; ++v) best = (kv[v] == kmax && cr[v] < best) ? cr[v] : best;
-      kmax = ((unsigned long long)(unsigned)uni((int)(kmax >> 32)) << 32) |
-             (unsigned)uni((int)(kmax & 0xffffffffull));
-      best = uni(best);
-      bc = best >> 7;
-      brow = best & 127;
-      par ^= 1;
-      const double vmax = __longlong_as_double((long long)kmax);
-      if (!(vmax >= fp.small) || bc >= 64 || brow >= 64) {
-        zero_rest(-5);
-        break;
-      }
-    }
-    // ---- owners broadcast their columns: cs[0] <- column bc, cs[1] <- column brow
-    if (lane == bc || lane == brow) {
-      double *dst = cs[lane == bc ? 0 : 1] + r0;
-#pragma unroll
-      for (int r = 0; r < R; ++r) dst[r] = a[r];
-    }
-    __syncthreads();
-    if (fp.posdef && !(uni(cs[0][bc]) > 0.0)) {
-      zero_rest(-6);
-      break;
-    }
-    int size, p1, p2 = -1;
-    const double *c1p, *c2p = cs[1];
-    double d11 = 0.0, d21 = 0.0, d22 = 0.0;
-    if (brow == bc) {
-      size = 1;
-      p1 = bc;
-      c1p = cs[0];
-    } else {
-      const double a11 = uni(cs[0][bc]), a22 = uni(cs[1][brow]), a21 = uni(cs[0][brow]);
-      // explicit fma throughout the block (no contraction left to the
-      // compiler), so the oracle's restatement can round the same way
-      const double detscale = 1.0 / fabs(a21);
-      const double detpiv = fma(a11 * detscale, a22, -fabs(a21));
-      if (fabs(detpiv) >= fabs(a21) / 2) {
-        size = 2;
-        p1 = bc;
-        p2 = brow;
-        c1p = cs[0];
-        d11 = (a22 * detscale) / detpiv;
-        d21 = (-a21 * detscale) / detpiv;
-        d22 = (a11 * detscale) / detpiv;
-      } else {
-        size = 1;
-        const bool first = fabs(a11) > fabs(a22);
-        p1 = first ? bc : brow;
-        c1p = first ? cs[0] : cs[1];
-      }
-    }
-    if (size == 1) {
-      const double di = 1.0 / c1p[p1];
-      elim |= 1ull << p1;
-      const double lj = c1p[lane] * di;  // L(lane, k)
-#pragma unroll
-      for (int r = 0; r < R; ++r) a[r] = fma(-c1p[r0 + r], lj, a[r]);
-      if (wv == 0) t[k][lane] = lj;
-      if (tid == 0) {
-        dinv[2 * k] = di;
-        dinv[2 * k + 1] = 0.0;
-        lp[k] = p1;
-        kind[k] = 1;
-      }
-    } else {
-      elim |= (1ull << p1) | (1ull << p2);
-      const double x = c1p[lane], y = c2p[lane];
-      const double l1 = fma(d11, x, d21 * y), l2 = fma(d21, x, d22 * y);
-#pragma unroll
-      for (int r = 0; r < R; ++r) a[r] = fma(-c1p[r0 + r], l1, fma(-c2p[r0 + r], l2, a[r]));
-      if (wv == 0) {
-        t[k][lane] = l1;
-        t[k + 1][lane] = l2;
-      }
-      if (tid == 0) {
-        dinv[2 * k] = d11;
-        dinv[2 * k + 1] = d21;
-        dinv[2 * k + 2] = INFINITY;
-        dinv[2 * k + 3] = d22;
-        lp[k] = p1;
-        lp[k + 1] = p2;
-        kind[k] = 2;
-        kind[k + 1] = 3;
-      }
-    }
-    k += size;
   }
+  if (stop != 0)
+    for (int kk = k + wv; kk < w; kk += NW) t[kk][lane] = 0.0;
   __syncthreads();
-  // ---- write back L_bb (rows permuted into elimination order), D^{-1}, lp
-  for (int i = tid; i < w; i += 64 * NW) inv_lp[lp[i]] = i;
-  __syncthreads();
-  for (int idx = tid; idx < w * w; idx += 64 * NW) {
-    const int r = idx % w, kk = idx / w;  // original row r, elimination column kk
-    const int nr = inv_lp[r];
-    if (nr < kk) continue;
-    double v;
-    if (nr == kk) v = (kind[kk] == 0) ? 0.0 : 1.0;
-    else if (nr == kk + 1 && kind[kk] == 2) v = 0.0;
-    else v = t[kk][r];
-    L[(size_t)(p + kk) * ldl + p + nr] = v;
+  // ---- write back L_bb (rows permuted into elimination order), D^{-1}, lp;
+  // mi[k][i] = L_bb[i][k], the strict lower part in elimination order
+  {
+    const int li = (lane < w) ? lp[lane] : 0, ki = (lane < w) ? kind[lane] : 0;
+    const unsigned long long two = __builtin_amdgcn_ballot_w64(ki == 2);
+    const unsigned long long zero = __builtin_amdgcn_ballot_w64(ki == 0);
+    gdouble *Lw = (gdouble *)L;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int kk = c0 + j;  // elimination column kk, row `lane`
+      const bool low = lane > kk && lane < w && !(lane == kk + 1 && ((two >> kk) & 1));
+      const double v = masked(t[kk][li], low);
+      mi[kk][lane] = v;
+      if (lane >= kk && lane < w)
+        Lw[(size_t)(p + kk) * ldl + p + lane] = (lane == kk) ? (((zero >> kk) & 1) ? 0.0 : 1.0) : v;
+    }
   }
   for (int j = tid; j < w; j += 64 * NW) {
     N.D[2 * (p + j)] = dinv[2 * j];
     N.D[2 * (p + j) + 1] = dinv[2 * j + 1];
     N.lp[j] = lp[j];
   }
-  // ---- M = L_bb^{-1} in elimination order for k_apply
-  // (L21 = A21[:, lp] M^T D^{-1}).  mi[k][i] = L_bb[i][k] (zero outside the
-  // strict lower w x w part), then forward substitution by columns: once
-  // m[k] is final it updates every later m[i]
-  for (int idx = tid; idx < kBlk * kBlk; idx += 64 * NW) {
-    const int i = idx & (kBlk - 1), k = idx / kBlk;
-    double v = 0.0;
-    if (i > k && i < w && !(kind[k] == 2 && i == k + 1)) v = t[k][lp[i]];
-    mi[k][i] = v;
-  }
   __syncthreads();
-  {
-    // wave v: columns [Cv, Cv+C) (C = 64/NW); NW lanes per column: lane =
-    // NW * (column in wave) + phase, rows phase, phase+NW, ... in registers
-    constexpr int C = kBlk / NW;
-    static_assert((NW & (NW - 1)) == 0 && C * NW == kBlk, "NW: a power of two");
-    const int col = wv * C + lane / NW, ph = lane % NW;
-    double mm[C];
-#pragma unroll
-    for (int q = 0; q < C; ++q) mm[q] = (ph + NW * q == col) ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 0; k < kBlk - 1; ++k) {
-      const double mk = __shfl(mm[k / NW], (lane & ~(NW - 1)) | (k % NW));
-#pragma unroll
-      for (int q = 0; q < C; ++q)
-        if (ph + NW * q > k) mm[q] -= mi[k][ph + NW * q] * mk;
-    }
-#pragma unroll
-    for (int q = 0; q < C; ++q) N.W[(ph + NW * q) * kBlk + col] = mm[q];  // row-major
-  }
+  block_inverse(mi, t, wv, lane, (gdouble *)N.W);
   // permute the variable list (rows of earlier eliminated columns: k_apply)
   const int pv = (tid < w) ? N.perm[p + lp[tid]] : 0;
   __syncthreads();
@@ -1889,11 +2126,11 @@ void launch_gather_first(hipStream_t st, int nwg, NodeDev *nodes, const int *slo
   const GatherArgs ga{wg_off, nlvl, child_list, aval, asrc, arow, acix, scaling};
   if (nwg <= 0) return;
   if (fp.c32)
-    hipLaunchKernelGGL((k_diag<kDiagWaves, true, true>), dim3(nwg), dim3(kThreads), 0, st,
-                       nodes, slots, 0, fp, ga);
+    hipLaunchKernelGGL((k_diag<kDiagWaves, true, true>), dim3(nwg), dim3(64 * kDiagWaves), 0,
+                       st, nodes, slots, 0, fp, ga);
   else
-    hipLaunchKernelGGL((k_diag<kDiagWaves, true, false>), dim3(nwg), dim3(kThreads), 0, st,
-                       nodes, slots, 0, fp, ga);
+    hipLaunchKernelGGL((k_diag<kDiagWaves, true, false>), dim3(nwg), dim3(64 * kDiagWaves), 0,
+                       st, nodes, slots, 0, fp, ga);
 }
 void launch_gather(hipStream_t st, int part, int nwg, NodeDev *nodes, const int *slots,
                    const int *wg_off, int nlvl, const int *child_list, const double *aval,
