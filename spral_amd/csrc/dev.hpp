@@ -56,7 +56,7 @@ struct NodeDev {
   int flag;         // 0 ok, -5 singular (action false)
   int nzero;
   int lp[kBlk];
-  unsigned long long colmax[kBlk];
+  unsigned long long fail;  // columns of the step's block with an |l| above 1/u
 };
 
 // Per-node view used by the solve kernels.

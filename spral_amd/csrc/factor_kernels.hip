@@ -12,7 +12,7 @@
 //               block with complete pivoting (1x1/2x2) in registers
 //               (pivot rules of src/ssids/cpu/kernels/block_ldlt.hxx:213-414).
 //  k_apply      L = A Lbb^{-T} D^{-1} for the rows below the block, keeping a
-//               backup and the column max |l| (a posteriori test,
+//               backup and the columns with an |l| > 1/u (a posteriori test,
 //               src/ssids/cpu/kernels/ldlt_app.cxx:304-414).
 //  k_update     restore failed columns and apply the accepted pivots to the
 //               trailing panel columns with v_mfma_f64_16x16x4_f64 on 64x64
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
 #pragma unroll
     for (int j = 0; j < R; ++j) t[lane][c0 + j] = v[j];
   }
-  if (tid < kBlk) N.colmax[tid] = 0ull;
+  if (tid == 0) N.fail = 0ull;
   __syncthreads();
   double16_t a;   // columns c0 .. c0 + 15 of row `lane`, zero outside the block
   uint16v_t msk;  // high-word mask of the search (0 above the diagonal)
@@ -643,16 +643,22 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
 }
 
 // ---------------------------------------------------------------------------
-// Apply the block pivots to the rows below and record column maxima
+// Apply the block pivots to the rows below and record the columns that fail
+// the a posteriori test.
+// The MFMA's output rows are the pivots and its columns the front's rows, so
+// a store covers four columns of 16 consecutive rows (whole lines) straight
+// from the accumulators; the block inverse is lower triangular, so pivot
+// block g takes 4 (g + 1) of the 16 pivot steps.  A column's largest |l| only
+// matters against 1/u: lanes compare, a wave's failures go to one 64-bit mask
+// by a ballot, and a workgroup without a failure writes none.  (With the
+// maxima kept as values, each workgroup reduced 64 columns by shuffles and
+// made 256 atomics on the front's 64 words.)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_apply(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int *lvl_slots,
                                                     const int *wg_off, int nlvl, int step,
                                                     FactorParams fp) {
-  // M = L_bb^{-1} (or the left-rows chunk), then, once the MFMAs have read
-  // it, X = A21[:, lp] M^T for this workgroup's 64 rows (one tile of LDS:
-  // four workgroups fit a CU)
+  // M = L_bb^{-1} (or the left-rows chunk)
   __shared__ double ms[kBlk][kBlk + 1];
-  double (*xs)[kBlk + 1] = ms;
   __shared__ double dv[2 * kBlk + 2];
   __shared__ int lps[kBlk];
   const int li = find_node(wg_off, nlvl, blockIdx.x);
@@ -671,29 +677,41 @@ __global__ __launch_bounds__(kThreads) void k_apply(NodeDev *nodes, const int *l
   if (local < nleft) {
     const int cb = local * kBlk;
     if (cb >= p) return;
-    for (int idx = tid; idx < kBlk * kBlk; idx += kThreads) {
-      int r = idx % kBlk, cc = idx / kBlk;
-      if (r < w && cb + cc < p) ms[r][cc] = L[(size_t)(cb + cc) * ldl + p + r];
-    }
+    gdouble *Lg = (gdouble *)L;
+    const int r = lane;
+    double v[kBlk / 4];
+#pragma unroll
+    for (int u = 0; u < kBlk / 4; ++u)
+      v[u] = Lg[(size_t)imin(cb + wave + 4 * u, p - 1) * ldl + p + imin(r, w - 1)];
+#pragma unroll
+    for (int u = 0; u < kBlk / 4; ++u) ms[r][wave + 4 * u] = v[u];
+    const int lr = N.lp[imin(r, w - 1)];
     __syncthreads();
-    for (int idx = tid; idx < kBlk * kBlk; idx += kThreads) {
-      int r = idx % kBlk, cc = idx / kBlk;
-      if (r < w && cb + cc < p) L[(size_t)(cb + cc) * ldl + p + r] = ms[N.lp[r]][cc];
+#pragma unroll
+    for (int u = 0; u < kBlk / 4; ++u) {
+      const int cc = wave + 4 * u;
+      if (r < w && cb + cc < p) Lg[(size_t)(cb + cc) * ldl + p + r] = ms[lr][cc];
     }
     return;
   }
   local -= nleft;
-  // ---- rows [rb, rb+64) below the block: X = A21[:, lp] M^T on MFMA
+  // ---- rows [rb, rb+64) below the block: X^T = M A21[:, lp]^T on MFMA
   const int r0 = p + w, m = N.m;
   const int rb = r0 + local * kBlk;
-  for (int idx = tid; idx < kBlk * kBlk; idx += kThreads)
-    ms[idx / kBlk][idx & (kBlk - 1)] = N.W[idx];
-  for (int j = tid; j < 2 * w; j += kThreads) dv[j] = N.D[2 * p + j];
+  if (rb >= m) return;
+  gcdouble *Wg = (gcdouble *)N.W;
+  gcdouble *Dg = (gcdouble *)N.D;
+  gcint *lpg = (gcint *)N.lp;
+  double wv[kBlk / 4];
+#pragma unroll
+  for (int u = 0; u < kBlk / 4; ++u) wv[u] = Wg[tid + u * kThreads];
+  if (tid < kBlk) lps[tid] = lpg[imin(tid, w - 1)];
+  else if (tid >= 2 * kBlk && tid < 4 * kBlk && tid - 2 * kBlk < 2 * w)
+    dv[tid - 2 * kBlk] = Dg[2 * p + tid - 2 * kBlk];
   if (tid == 0) {
     dv[2 * w] = 0.0;
     dv[2 * w + 1] = 0.0;
   }
-  for (int j = tid; j < kBlk; j += kThreads) lps[j] = (j < w) ? N.lp[j] : 0;
   __syncthreads();
   const int ri = lane & 15, kq = lane >> 4;
   const int r = rb + wave * 16 + ri;  // A row of this lane (fragment layout)
@@ -705,16 +723,19 @@ __global__ __launch_bounds__(kThreads) void k_apply(NodeDev *nodes, const int *l
 #pragma unroll
     for (int u = 0; u < kBlk / 4; ++u) {
       const int k = 4 * u + kq;
-      av[u] = masked(Lg[(size_t)(p + lps[imin(k, w - 1)]) * ldl + rc], rok && k < w);
+      av[u] = masked(Lg[(size_t)(p + lps[k]) * ldl + rc], rok && k < w);
     }
   }
+#pragma unroll
+  for (int u = 0; u < kBlk / 4; ++u)
+    ms[(tid + u * kThreads) / kBlk][tid & (kBlk - 1)] = wv[u];
   // descriptor fields once: the global stores below could otherwise alias
   // them and force a reload per iteration
   gdouble *bak = (gdouble *)N.bak;
   gdouble *LD = (gdouble *)N.LD;
   gdouble *Lw = (gdouble *)L;
-  unsigned long long *colmax = N.colmax;
   const int ldbak = N.ldbak, nfs = N.n;
+  __syncthreads();
 #pragma unroll
   for (int u = 0; u < kBlk / 4; ++u) {
     const int k = 4 * u + kq;
@@ -726,72 +747,68 @@ __global__ __launch_bounds__(kThreads) void k_apply(NodeDev *nodes, const int *l
 #pragma unroll
   for (int u = 0; u < kBlk / 4; ++u) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g)  // B[k][j] = M[j][k]
-      acc[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], ms[g * 16 + ri][4 * u + kq], acc[g],
+    for (int g = u / 4; g < 4; ++g)  // A[j][k] = M[j][k], zero for k > j
+      acc[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(ms[g * 16 + ri][4 * u + kq], av[u], acc[g],
                                                     0, 0, 0);
   }
-  __syncthreads();  // every wave has read M before X overwrites it
+  // ---- x D^{-1}: acc[g][q] is row r, pivot j = 16 g + 4 q + kq
+  const double lim = 1.0 / fp.u;
+  // the partner of a 2x2 pivot is one lane group up (down), or the next
+  // (previous) register's first (last) group; uniform over the workgroup
+  bool two = false;
+  for (int j = lane; j < w; j += 64) two = isinf(dv[2 * j]);
+  two = __builtin_amdgcn_ballot_w64(two) != 0ull;
+  const int up = (lane + 16) & 63, dn = (lane - 16) & 63;
+  double nx[17], pvx[17];
+  if (two) {
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
+    for (int i = 0; i < 16; ++i) {
+      nx[i] = __shfl(acc[i / 4][i % 4], up);
+      pvx[i + 1] = __shfl(acc[i / 4][i % 4], dn);
+    }
+    nx[16] = 0.0;
+    pvx[0] = 0.0;
+  }
+  unsigned long long fail = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) xs[wave * 16 + 4 * q + kq][g * 16 + ri] = acc[g][q];
-  __syncthreads();
-  // ---- x D^{-1}, store, column maxima (thread: row `row`, columns cb0 + 4u)
-  const int row = lane, cb0 = wave;
-  const int rr = rb + row;
-  const bool ok = rr < m;
-  const double small = fp.small;
-#pragma unroll
-  for (int u = 0; u < kBlk / 4; ++u) {
-    const int j = cb0 + 4 * u;
-    double y = 0.0;
-    if (j < w) {
-      const double xj = xs[row][j];
-      const bool two_first = (j + 1 < w) && isinf(dv[2 * j + 2]);
-      const bool two_second = (j > 0) && isinf(dv[2 * j]);
-      bool zero_piv = false;
-      if (two_first) {
-        y = dv[2 * j] * xj + dv[2 * j + 1] * xs[row][j + 1];
-      } else if (two_second) {
-        y = dv[2 * j - 1] * xs[row][j - 1] + dv[2 * j + 1] * xj;
-      } else {
-        const double d11 = dv[2 * j];
-        zero_piv = (d11 == 0.0);
-        if (zero_piv) y = (fabs(xj) < small) ? 0.0 : INFINITY * xj;
-        else y = xj * d11;
-      }
-      if (ok) {
-        Lw[(size_t)(p + j) * ldl + rr] = y;
-        // L21 D is the product before D^{-1} (zero for a zero pivot): the
-        // parent's gather operand, for the contribution rows
-        if (LD && rr >= nfs) LD[(size_t)(p + j) * ldl + rr] = zero_piv ? 0.0 : xj;
+  for (int i = 0; i < 16; ++i) {
+    const int j = 4 * i + kq;
+    const double xj = acc[i / 4][i % 4];
+    const double d11 = dv[2 * imin(j, w)];
+    double y = xj * d11;
+    bool zero_piv = d11 == 0.0;
+    if (zero_piv) y = (fabs(xj) < fp.small) ? 0.0 : INFINITY * xj;
+    if (two) {
+      const double xn = kq < 3 ? nx[i] : nx[i + 1], xp = kq > 0 ? pvx[i + 1] : pvx[i];
+      if (j + 1 < w && isinf(dv[2 * j + 2])) {
+        y = d11 * xj + dv[2 * j + 1] * xn;
+        zero_piv = false;
+      } else if (j > 0 && j < w && isinf(d11)) {
+        y = dv[2 * j - 1] * xp + dv[2 * j + 1] * xj;
       }
     }
-    // column maximum over this wave's 64 rows (NaN propagates as a failure)
-    double v = (ok && j < w) ? fabs(y) : 0.0;
-    for (int off = 32; off > 0; off >>= 1) {
-      const double o = __shfl_xor(v, off);
-      v = (o > v || isnan(o)) ? o : v;
+    const bool ok = rok && j < w;
+    if (ok) {
+      Lw[(size_t)(p + j) * ldl + r] = y;
+      // L21 D is the product before D^{-1} (zero for a zero pivot): the
+      // parent's gather operand, for the contribution rows
+      if (LD && r >= nfs) LD[(size_t)(p + j) * ldl + r] = zero_piv ? 0.0 : xj;
     }
-    if (lane == 0 && j < w) {
-      const unsigned long long bits = isnan(v) ? 0x7ff0000000000001ull
-                                               : (unsigned long long)__double_as_longlong(v);
-      atomicMax(&colmax[j], bits);
+    // a NaN fails too
+    unsigned long long f = __builtin_amdgcn_ballot_w64(ok && !(fabs(y) <= lim));
+    if (f) {  // bit 16 k' + row: pivot 4 i + k'
+      for (int k = 0; k < 4; ++k)
+        if ((f >> (16 * k)) & 0xffffull) fail |= 1ull << (4 * i + k);
     }
   }
+  if (fail && lane == 0) atomicOr(&N.fail, fail);
 }
 
 // number of block pivots that pass the threshold test (split 2x2 avoided):
-// the first column whose max |l| exceeds 1/u.  Lane j reads column j's
-// maximum, so the w loads are in flight together; every lane of the wave
-// must be active, and the result is wave-uniform.
-__device__ inline int block_npass(const NodeDev &N, double u) {
-  const int w = N.w, p = N.p, lane = threadIdx.x & 63;
-  const double lim = 1.0 / u;
-  const unsigned long long lb = (unsigned long long)__double_as_longlong(lim);
-  const unsigned long long b =
-      (lane < w) ? __atomic_load_n(&N.colmax[lane], __ATOMIC_RELAXED) : 0ull;
-  const unsigned long long fail = __ballot(lane < w && b > lb);
+// the first column holding an |l| above 1/u; wave-uniform.
+__device__ inline int block_npass(const NodeDev &N) {
+  const int w = N.w, p = N.p;
+  const unsigned long long fail = __atomic_load_n(&N.fail, __ATOMIC_RELAXED);
   int np = fail ? __ffsll((long long)fail) - 1 : w;
   if (np > 0 && np < w) {
     double d11 = N.D[2 * (p + np - 1)], d21 = N.D[2 * (p + np - 1) + 1];
@@ -864,7 +881,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, const in
     p = N.p;
     w = N.w;
     if (w == 0) return;
-    int np = fp.posdef ? N.w : block_npass(N, fp.u);
+    int np = fp.posdef ? N.w : block_npass(N);
     if (local == 0 && tid == 0) N.npass = np;
     a0 = p;
     K = np;
@@ -1006,7 +1023,7 @@ __global__ __launch_bounds__(kThreads, 3) void k_update_panel(NodeDev *nodes,
   if (step >= N.nsteps) return;
   const int p = N.p, w = N.w;
   if (w == 0) return;
-  const int np = fp.posdef ? w : block_npass(N, fp.u);
+  const int np = fp.posdef ? w : block_npass(N);
   if (local == 0 && tid == 0) N.npass = np;
   const int a0 = p, K = np, t0 = p + np, cend = N.n, fa = p + np, fb = p + w;
   const int m = N.m;
