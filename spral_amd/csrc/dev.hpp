@@ -37,7 +37,6 @@ struct NodeDev {
   double *dbak;     // kBlk x kBlk backup of the diagonal block
   double *W;        // kBlk x kBlk row-major: inverse of the step's unit lower
                     // diagonal block (elimination order), for k_apply
-  double *swp;      // 2*kBlk x m gather buffer for the failed-column swap
   int *pmap;        // (m - nelim) parent positions of the trailing indices
   int *ctab;        // per child (stride T+1, T = 64-row tiles of this front):
                     // tile t -> first child trailing index mapping to >= 64t

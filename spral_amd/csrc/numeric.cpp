@@ -41,7 +41,7 @@ void launch_apply(hipStream_t, int, NodeDev *, const int *, const int *, int, in
                   FactorParams);
 void launch_update(hipStream_t, int, NodeDev *, const int *, const int *, int, int, int,
                    FactorParams);
-void launch_swap(hipStream_t, int, NodeDev *, const int *, const int *, int, int, int);
+void launch_swap(hipStream_t, int, NodeDev *, const int *, const int *, int, int);
 void launch_tail(hipStream_t, int, NodeDev *, const int *, FactorParams, int *);
 void launch_stats(hipStream_t, const NodeDev *, int, int *, const FactorParams &);
 void launch_level_setup(hipStream_t, NodeDev *, int, int, const int *, int, int, int *, int *);
@@ -248,7 +248,6 @@ struct Plan {
   NodeDev *d_tmpl = nullptr;
   struct Level {
     int maxsteps = 0;
-    bool multi = false;
     size_t tab_off = 0;
     std::vector<int> cap;                   // capacity workgroups per table
   };
@@ -584,12 +583,11 @@ static void set_contrib(NodeDev &D, char *base, size_t cbytes, size_t ldbytes) {
   D.C = (D.ldc > 0) ? (double *)base : nullptr;
   D.LD = ldbytes ? (double *)(base + cbytes) : nullptr;
 }
-// The APP workspace: backups, the block inverse, the swap buffer
+// The APP workspace: backups and the block inverse
 static void set_work(NodeDev &D, char *w, int nsteps) {
   D.bak = (double *)w;
   D.dbak = D.bak + (size_t)D.ldbak * kBlk;
   D.W = D.dbak + kBlk * kBlk;
-  D.swp = (nsteps > 1) ? D.W + kBlk * kBlk : nullptr;
 }
 
 // Bytes of a front's transient blocks (D.ldl, D.ldc, D.ldbak set): the
@@ -601,7 +599,6 @@ static void trans_sizes(const Numeric &N, const NodeDev &D, int n, int nsteps, i
   cbytes = ((size_t)D.ldc * (D.sm - D.sn) * cesz + 255) & ~size_t(255);
   ldbytes = D.is_root ? 0 : (size_t)D.ldl * n * sizeof(double);
   wb = ((size_t)D.ldbak * kBlk + 2 * kBlk * kBlk) * sizeof(double);
-  if (nsteps > 1) wb += (size_t)2 * kBlk * m * sizeof(double);
 }
 
 // Buffers of a front with room for m rows / n fully-summed columns.
@@ -768,7 +765,6 @@ static void plan_build(Numeric &N, int pivot_tpp, double multiplier) {
       nc[sl - s0] = n;
       sc[sl - s0] = nsteps;
       lv.maxsteps = std::max(lv.maxsteps, nsteps);
-      if (nsteps > 1) lv.multi = true;
       cur_sl = sl;
       node_buffers(N, S, sl, D, m, n, nsteps, keep, trans, cof[sl], wof[sl]);
     }
@@ -889,10 +885,9 @@ static bool factor_static(Numeric &N, const FactorParams &fp, const spral_ssids_
       if (ms > 1) join();
       launch_update(st, lv.cap[ms + 2 + stp], N.d_nodes, d_slots, toff(ms + 2 + stp), nl, stp,
                     0, fp);
-      if (lv.multi) {
-        launch_swap(st, lv.cap[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp, 0);
-        launch_swap(st, lv.cap[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp, 1);
-      }
+      // (the last step leaves no unprocessed candidate to swap with)
+      if (stp + 1 < ms)
+        launch_swap(st, lv.cap[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp);
     }
     join();
     launch_tail(st, nl, N.d_nodes, d_slots, fp, N.d_scratch_n);
@@ -998,7 +993,6 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
   for (int L = 0; L < nlev; ++L) {
     const int s0 = S.lvl_ptr[L], s1 = S.lvl_ptr[L + 1], nl = s1 - s0;
     int maxsteps = 0;
-    bool multi = false;
     for (int sl = s0; sl < s1; ++sl) {
       const int i = S.node_of[sl];
       NodeDev &D = N.nodes[sl];
@@ -1015,7 +1009,6 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
       D.n = D.sn + nd;
       D.nsteps = fp.pivot_tpp ? 0 : cdiv(D.n, kBlk);
       maxsteps = std::max(maxsteps, D.nsteps);
-      if (D.nsteps > 1) multi = true;
       node_buffers(N, S, sl, D, D.m, D.n, D.nsteps, keep,
                    [&](size_t b, int) { return N.pool.alloc(b); }, contrib_of[sl],
                    work_of[sl]);
@@ -1054,10 +1047,8 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
       launch_apply(st, tot[1 + stp], N.d_nodes, d_slots, toff(1 + stp), nl, stp, fp);
       launch_update(st, tot[ms + 2 + stp], N.d_nodes, d_slots, toff(ms + 2 + stp), nl, stp, 0,
                     fp);
-      if (multi) {
-        launch_swap(st, tot[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp, 0);
-        launch_swap(st, tot[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp, 1);
-      }
+      if (stp + 1 < ms)
+        launch_swap(st, tot[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp);
     }
     launch_tail(st, nl, N.d_nodes, d_slots, fp, N.d_scratch_n);
     if (tot[2 * ms + 2] > 0)
