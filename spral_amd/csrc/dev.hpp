@@ -7,7 +7,7 @@ namespace ssids_hip {
 
 constexpr int kBlk = 64;        // APP pivot block width (columns per step)
 constexpr int kThreads = 256;   // threads per workgroup in most kernels
-// least workgroups of a large front's APP trailing update (two per CU)
+// workgroups of a large front's APP trailing update (two per CU)
 constexpr int kUpdMinWgs = 512;
 
 // Per-node descriptor, stored contiguously in tree-level order ("slots").
@@ -37,6 +37,8 @@ struct NodeDev {
   double *dbak;     // kBlk x kBlk backup of the diagonal block
   double *W;        // kBlk x kBlk row-major: inverse of the step's unit lower
                     // diagonal block (elimination order), for k_apply
+  double *X;        // (m x kBlk, ld ldbak) L21 D of the step's pivots for the
+                    // fully-summed rows below the block
   int *pmap;        // (m - nelim) parent positions of the trailing indices
   int *ctab;        // per child (stride T+1, T = 64-row tiles of this front):
                     // tile t -> first child trailing index mapping to >= 64t
@@ -122,15 +124,13 @@ __host__ __device__ inline int level_table_count(int t, int S, int m, int n, int
   if (t <= 2 * S + 1) {
     const int stp = t - S - 2;
     if (stp >= nsteps) return 0;
-    const int t0 = imin(n, (stp + 1) * kBlk);
-    const int TI = idiv_up(m - t0, kBlk), TJ = idiv_up(n - t0, kBlk);
-    const int nt = TJ * TI - TJ * (TJ - 1) / 2;
-    // the count above assumes every earlier pivot passed; failed columns
-    // leave a larger trailing panel (down to the whole front), which the
-    // workgroups stride over, so a large front keeps at least kUpdMinWgs
+    // two workgroups fit a CU, and a workgroup's run of tiles costs less than
+    // as many workgroups of one tile, so a front gets at most kUpdMinWgs.
+    // The whole front's tiles bound the step's: failed columns leave a larger
+    // trailing panel than the step's number says
     const int TM = idiv_up(m, kBlk), TN = idiv_up(n, kBlk);
     const int nt_all = TN * TM - TN * (TN - 1) / 2;
-    return imax(1, imax(imin(nt, 4096), imin(nt_all, kUpdMinWgs)));
+    return imax(1, imin(nt_all, kUpdMinWgs));
   }
   if (t == 2 * S + 2) {
     if (!is_root || m <= n) return 0;

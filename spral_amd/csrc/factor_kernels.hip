@@ -733,6 +733,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int
   // them and force a reload per iteration
   gdouble *bak = (gdouble *)N.bak;
   gdouble *LD = (gdouble *)N.LD;
+  gdouble *X = (gdouble *)N.X;
   gdouble *Lw = (gdouble *)L;
   const int ldbak = N.ldbak, nfs = N.n;
   __syncthreads();
@@ -791,8 +792,11 @@ __global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int
     if (ok) {
       Lw[(size_t)(p + j) * ldl + r] = y;
       // L21 D is the product before D^{-1} (zero for a zero pivot): the
-      // parent's gather operand, for the contribution rows
-      if (LD && r >= nfs) LD[(size_t)(p + j) * ldl + r] = zero_piv ? 0.0 : xj;
+      // trailing update's operand for the fully-summed rows, the parent's
+      // gather operand for the contribution rows
+      const double x = zero_piv ? 0.0 : xj;
+      if (r < nfs) X[(size_t)j * ldbak + (r - r0)] = x;
+      else if (LD) LD[(size_t)(p + j) * ldl + r] = x;
     }
     // a NaN fails too
     unsigned long long f = __builtin_amdgcn_ballot_w64(ok && !(fabs(y) <= lim));
@@ -852,15 +856,17 @@ __device__ inline void pivot_d(const double *D, int k, int kend, double &e1, dou
 // ---------------------------------------------------------------------------
 constexpr int kTile = 64;
 
+// lower tiles (I >= J), column-major over J: column J starts at
+// J TI - J (J - 1) / 2.  The root of that quadratic in single precision is at
+// most a column off, which the two loops correct.
 __device__ inline void tile_of(int tile, int TI, int TJ, int &I, int &J) {
-  // lower tiles (I >= J), column-major over J
-  int t = tile;
-  J = 0;
-  while (J < TJ && t >= TI - J) {
-    t -= TI - J;
-    ++J;
-  }
-  I = J + t;
+  auto first = [&](int j) { return j * TI - j * (j - 1) / 2; };
+  const float h = 2.0f * (float)TI + 1.0f;
+  J = (int)(0.5f * (h - __builtin_sqrtf(fmaxf(h * h - 8.0f * (float)tile, 0.0f))));
+  J = imax(0, imin(J, TJ - 1));
+  while (J > 0 && first(J) > tile) --J;
+  while (J + 1 < TJ && first(J + 1) <= tile) ++J;
+  I = J + (tile - first(J));
 }
 
 __global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, const int *lvl_slots,
@@ -998,18 +1004,128 @@ __global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, const in
 
 // ---------------------------------------------------------------------------
 // The APP step's trailing panel update (k_update mode 0) with the MFMA
-// operands loaded straight into the 16x16x4 fragment layout: lane i + 16 kq
-// holds row i of A (= L, pivot kq of the 4-pivot step) and column i of
-// B = L D for the same pivot; two register buffers of two steps each
-// alternate, so the loads of the next 8 pivots are in flight during the
-// MFMAs.  The per-pivot coefficients of L D come from pivot_d once per
-// workgroup.  Each element gets the same products in the same order as in
-// k_update.  Three workgroups per SIMD fit (162 VGPRs): loading the tile's
-// current values before the products as well needs 198 registers and two
-// workgroups, and measured slower (64^3 factor 47.4 against 46.7 ms, the
-// LDS-staged k_update 48.1 ms).
+// operands loaded straight into the 16x16x4 fragment layout.
+//
+// A step whose 64-column block passed whole (nearly every step of a
+// well-ordered matrix): update_tiles.  Output rows are the panel's columns and
+// output columns its rows, so a load or store of the panel covers four
+// columns of 16 consecutive rows (whole lines).  L D is the apply's product
+// before D^{-1}, stored by it (X), so no coefficients or 2x2 partners are
+// needed.  A workgroup takes a run of consecutive tiles (column by column);
+// all of a tile's loads are out before its products, and each operand
+// register is reloaded for the next tile right after its last use, so a tile
+// costs its products and not the memory latency.
+//
+// Other steps (failed columns, a last narrower block): lane i + 16 kq holds row i of A (= L, pivot kq of
+// the 4-pivot step) and column i of B = L D for the same pivot; two register
+// buffers of two steps each alternate, so the loads of the next 8 pivots are
+// in flight during the MFMAs.  The per-pivot coefficients of L D come from
+// pivot_d once per workgroup.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 3) void k_update_panel(NodeDev *nodes,
+// Addresses are a uniform base plus a 32-bit lane offset inside 64 columns.
+__device__ __forceinline__ double load_at(gcdouble *base, unsigned off) { return base[off]; }
+
+__device__ __forceinline__ void update_tiles(gdouble *NL, int ldl, gcdouble *X, int ldx, int p,
+                                             int m, int n, int TI, int TJ, int tile, int tend) {
+  const int t0 = p + kBlk;
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
+  const int ri = lane & 15, kq = lane >> 4;
+  const int wr = t0 + (wave >> 1) * 32, wc = (wave & 1) * 32;
+  int I, J;
+  tile_of(tile, TI, TJ, I, J);
+  I = uni(I);
+  J = uni(J);
+  gcdouble *Lp = (gcdouble *)NL + (size_t)p * ldl;
+  double xa[2][kBlk / 4], la[2][kBlk / 4], old[2][2][4];
+  unsigned lo[2], xo[2];  // lane offsets of the tile being loaded
+  int rn[2];              // its rows
+  auto place = [&](int I, int J) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      rn[b] = imin(wr + I * kTile + 16 * b + ri, m - 1);
+      lo[b] = (unsigned)(kq * ldl + rn[b]);
+      xo[b] = (unsigned)(kq * ldx + imin(t0 + J * kTile + wc + 16 * b + ri, n - 1) - t0);
+    }
+  };
+  auto load_x = [&](int u) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) xa[b][u] = load_at(X + (size_t)(4 * u) * ldx, xo[b]);
+  };
+  auto load_l = [&](int u) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) la[b][u] = load_at(Lp + (size_t)(4 * u) * ldl, lo[b]);
+  };
+  auto load_old = [&](int J) {
+    gcdouble *Cb = (gcdouble *)NL + (size_t)(t0 + J * kTile) * ldl;
+    const int cl = n - 1 - (t0 + J * kTile);  // last column of the tile column
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const int c = imin(wc + 16 * bi + kq + 4 * rg, cl);
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj)
+          old[bi][bj][rg] = load_at(Cb, (unsigned)(c * ldl + rn[bj]));
+      }
+  };
+  place(I, J);
+#pragma unroll
+  for (int u = 0; u < kBlk / 4; ++u) {
+    load_x(u);
+    load_l(u);
+  }
+  load_old(J);
+  while (true) {
+    // the next tile of the run
+    int In = I, Jn = J;
+    ++tile;
+    const bool more = tile < tend;
+    if (more) {
+      ++In;
+      if (In >= TI) In = ++Jn;
+    }
+    place(In, Jn);
+    double4_t acc[2][2];
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj) acc[bi][bj] = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < kBlk / 4; ++u) {
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj)
+          acc[bi][bj] =
+              __builtin_amdgcn_mfma_f64_16x16x4f64(xa[bi][u], la[bj][u], acc[bi][bj], 0, 0, 0);
+      if (more) load_l(u);
+    }
+    if (Jn != J) {
+#pragma unroll
+      for (int u = 0; u < kBlk / 4; ++u) load_x(u);
+    }
+    gdouble *Cb = NL + (size_t)(t0 + J * kTile) * ldl;
+    const int c0 = t0 + J * kTile, r0 = wr + I * kTile + ri;
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const int c = wc + 16 * bi + kq + 4 * rg;
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj) {
+          const int r = r0 + 16 * bj;
+          if (r < m && c0 + c < n && r >= c0 + c)
+            Cb[(unsigned)(c * ldl + r)] = old[bi][bj][rg] - acc[bi][bj][rg];
+        }
+      }
+    if (!more) break;
+    load_old(Jn);
+    I = In;
+    J = Jn;
+  }
+}
+
+__global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
                                                            const int *lvl_slots,
                                                            const int *wg_off, int nlvl,
                                                            int step, FactorParams fp) {
@@ -1030,6 +1146,22 @@ __global__ __launch_bounds__(kThreads, 3) void k_update_panel(NodeDev *nodes,
   if (m - t0 <= 0 || cend - t0 <= 0) return;
   const int TI = (m - t0 + kTile - 1) / kTile, TJ = (cend - t0 + kTile - 1) / kTile;
   const int ntiles = TJ * TI - TJ * (TJ - 1) / 2;
+  if (np == kBlk) {
+    gdouble *NL = (gdouble *)N.L;
+    gcdouble *X = (gcdouble *)N.X;
+    const int ldl = N.ldl, ldx = N.ldbak;
+    // a run of consecutive tiles each; workgroups go to the eight XCDs in
+    // turn, and the runs of one XCD's workgroups are neighbours, so that its
+    // L2 holds the operands of few tile columns
+    const int used = imin(count, ntiles);
+    if (local >= used) return;
+    const int c8 = used >> 3;
+    const int run = (local < 8 * c8) ? (local & 7) * c8 + (local >> 3) : local;
+    const int tb = (int)((int64_t)run * ntiles / used);
+    const int te = (int)((int64_t)(run + 1) * ntiles / used);
+    update_tiles(NL, ldl, X, ldx, p, m, cend, TI, TJ, tb, te);
+    return;
+  }
   {
     const double *D = N.D;
     for (int t = tid; t < K; t += kThreads) {

@@ -583,11 +583,12 @@ static void set_contrib(NodeDev &D, char *base, size_t cbytes, size_t ldbytes) {
   D.C = (D.ldc > 0) ? (double *)base : nullptr;
   D.LD = ldbytes ? (double *)(base + cbytes) : nullptr;
 }
-// The APP workspace: backups and the block inverse
+// The APP workspace: backups, the block inverse, the step's L21 D
 static void set_work(NodeDev &D, char *w, int nsteps) {
   D.bak = (double *)w;
   D.dbak = D.bak + (size_t)D.ldbak * kBlk;
   D.W = D.dbak + kBlk * kBlk;
+  D.X = D.W + kBlk * kBlk;
 }
 
 // Bytes of a front's transient blocks (D.ldl, D.ldc, D.ldbak set): the
@@ -598,7 +599,7 @@ static void trans_sizes(const Numeric &N, const NodeDev &D, int n, int nsteps, i
   const size_t cesz = N.c32 ? sizeof(float) : sizeof(double);
   cbytes = ((size_t)D.ldc * (D.sm - D.sn) * cesz + 255) & ~size_t(255);
   ldbytes = D.is_root ? 0 : (size_t)D.ldl * n * sizeof(double);
-  wb = ((size_t)D.ldbak * kBlk + 2 * kBlk * kBlk) * sizeof(double);
+  wb = ((size_t)D.ldbak * 2 * kBlk + 2 * kBlk * kBlk) * sizeof(double);
 }
 
 // Buffers of a front with room for m rows / n fully-summed columns.
