@@ -863,7 +863,7 @@ __device__ inline void tile_of(int tile, int TI, int TJ, int &I, int &J) {
   auto first = [&](int j) { return j * TI - j * (j - 1) / 2; };
   const float h = 2.0f * (float)TI + 1.0f;
   J = (int)(0.5f * (h - __builtin_sqrtf(fmaxf(h * h - 8.0f * (float)tile, 0.0f))));
-  J = imax(0, imin(J, TJ - 1));
+  J = uni(imax(0, imin(J, TJ - 1)));  // the tile number is the workgroup's
   while (J > 0 && first(J) > tile) --J;
   while (J + 1 < TJ && first(J + 1) <= tile) ++J;
   I = J + (tile - first(J));
@@ -1033,8 +1033,6 @@ __device__ __forceinline__ void update_tiles(gdouble *NL, int ldl, gcdouble *X, 
   const int wr = t0 + (wave >> 1) * 32, wc = (wave & 1) * 32;
   int I, J;
   tile_of(tile, TI, TJ, I, J);
-  I = uni(I);
-  J = uni(J);
   gcdouble *Lp = (gcdouble *)NL + (size_t)p * ldl;
   double xa[2][kBlk / 4], la[2][kBlk / 4], old[2][2][4];
   unsigned lo[2], xo[2];  // lane offsets of the tile being loaded
@@ -1319,6 +1317,31 @@ __global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, const int *
   }
 }
 
+// Guarded loads without branches: a buffer load whose byte offset is at or
+// past the buffer's length reads nothing and returns zero, so a lane that has
+// nothing to load takes the offset kNoLoad.  (As conditional expressions the
+// same loads became branches, and those of FP32 blocks waited for each value
+// in turn to convert it: 12 us of a tile's 30.)  The base and the length are
+// uniform; lengths stay below 2^31.
+constexpr unsigned kNoLoad = 0xfffffff0u;
+typedef unsigned uint2v_t __attribute__((ext_vector_type(2)));
+template <typename T>
+struct LoadBuffer {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ LoadBuffer(const T *base, int64_t bytes)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T *>(base), 0,
+            (int)(bytes < 0 ? 0 : bytes > 0x7fffffff ? 0x7fffffff : bytes), 0x00020000)) {}
+  __device__ T operator()(unsigned off) const {
+    if constexpr (sizeof(T) == 4) {
+      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
+    } else {
+      const uint2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0);
+      return __hiloint2double((int)v.y, (int)v.x);
+    }
+  }
+};
+
 // PART 0: every tile of the level's fronts; 1: the first tile column only
 // (the pivot block and the rows below it); 2: the remaining tiles
 // Returns the front's slot when this workgroup built the front's first
@@ -1407,14 +1430,13 @@ __device__ __forceinline__ int gather_tile(
     const NodeDev &c = nodes[child_list[ci]];
     const int cn = c.n, cm = c.m, kb = c.nelim, cldl = c.ldl, cldc = c.ldc;
     gcdouble *cL = (gcdouble *)c.L;
-    gcdouble *cLD = (gcdouble *)c.LD;
-    const CT __attribute__((address_space(1))) *cC =
-        (const CT __attribute__((address_space(1))) *)c.C;
+    const double *cLD = c.LD;
+    const CT *cC = (const CT *)c.C;
     gcint *cpmap = (gcint *)c.pmap;
     if (cm <= kb) continue;
     gcint *tab = pctab + (size_t)(ci - cbeg) * (T + 1);
-    const int kr0 = tab[I], kr1 = tab[I + 1];
-    const int k0 = tab[J], k1 = tab[J + 1];
+    const int kr0 = uni(tab[I]), kr1 = uni(tab[I + 1]);
+    const int k0 = uni(tab[J]), k1 = uni(tab[J + 1]);
     if (kr1 <= kr0 || k1 <= k0 || kr1 - 1 < k0) continue;
     for (int t = tid; t < kr1 - kr0; t += kThreads) mr[t] = cpmap[kr0 + t - kb] - r0;
     for (int t = tid; t < k1 - k0; t += kThreads) mc[t] = cpmap[k0 + t - kb] - c0;
@@ -1427,14 +1449,21 @@ __device__ __forceinline__ int gather_tile(
     const bool contrib = (k1 > kc0 && kr1 > rr0);
     // C_c, lower part, down its columns: all loads issued before any use
     constexpr int NU = kGT / (kThreads / 64);
-    double cv[NU];
+    CT cv[NU];
     const bool rowok = contrib && ta < nrow;
     const int kr = rr0 + ta;
-    const CT __attribute__((address_space(1))) *Cr = cC + (kr - cn);
+    // columns b < blim of this thread's row are in the lower part
+    const int blim = rowok ? imin(ncol, kr - kc0 + 1) : 0;
+    {
+      const LoadBuffer<CT> Cb(cC + (size_t)(kc0 - cn) * cldc,
+                              contrib ? (int64_t)kGT * cldc * sizeof(CT) : 0);
+      const unsigned co = (unsigned)(tb * cldc + (kr - cn)) * sizeof(CT);
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int b = tb + u * (kThreads / 64), k = kc0 + b;
-      cv[u] = (rowok && b < ncol && kr >= k) ? (double)Cr[(size_t)(k - cn) * cldc] : 0.0;
+      for (int u = 0; u < NU; ++u) {
+        const int b = tb + u * (kThreads / 64);
+        cv[u] = Cb(b < blim ? co + (unsigned)(u * (kThreads / 64) * cldc) * sizeof(CT)
+                            : kNoLoad);
+      }
     }
     // L21 (L21 D)^T on MFMA: each wave a 32x32 quadrant, operands in the
     // 16x16x4 fragment layout (lane i+16k holds row i, pivot k) straight
@@ -1443,8 +1472,10 @@ __device__ __forceinline__ int gather_tile(
     const int K = kb;
     const int ra0 = wr + ri, ra1 = ra0 + 16, cb0 = wc + ri, cb1 = cb0 + 16;
     const bool va0 = ra0 < nrow, va1 = ra1 < nrow, vb0 = cb0 < ncol, vb1 = cb1 < ncol;
-    gcdouble *La = cL + rr0;
-    gcdouble *Lb = cLD + kc0;
+    const unsigned oa0 = va0 ? (unsigned)(kq * cldl + rr0 + ra0) * 8u : kNoLoad;
+    const unsigned oa1 = va1 ? (unsigned)(kq * cldl + rr0 + ra1) * 8u : kNoLoad;
+    const unsigned ob0 = vb0 ? (unsigned)(kq * cldl + kc0 + cb0) * 8u : kNoLoad;
+    const unsigned ob1 = vb1 ? (unsigned)(kq * cldl + kc0 + cb1) * 8u : kNoLoad;
     // FP64: v_mfma_f64_16x16x4_f64, D[i][j] in lane j + 16 (i % 4), register
     // i / 4.  Mixed precision: operands rounded to FP32, v_mfma_f32_16x16x4_f32
     // with FP32 accumulation, D[i][j] in lane j + 16 (i / 4), register i % 4
@@ -1459,13 +1490,16 @@ __device__ __forceinline__ int gather_tile(
     auto load = [&](int T0, double *A0, double *A1, double *B0, double *B1) {
 #pragma unroll
       for (int u = 0; u < KC; ++u) {
-        const int t = T0 + 4 * u + kq;
-        const bool ok = t < K;
-        const size_t o = (size_t)t * cldl;
-        A0[u] = (ok && va0) ? La[o + ra0] : 0.0;
-        A1[u] = (ok && va1) ? La[o + ra1] : 0.0;
-        B0[u] = (ok && vb0) ? Lb[o + cb0] : 0.0;
-        B1[u] = (ok && vb1) ? Lb[o + cb1] : 0.0;
+        // the length ends with pivot K - 1: a lane whose pivot T + kq is past
+        // it loads nothing
+        const int T = T0 + 4 * u;
+        const int64_t left = (int64_t)(K - T) * cldl * 8;
+        const LoadBuffer<double> Lb((const double *)cL + (size_t)T * cldl, left);
+        const LoadBuffer<double> Db(cLD + (size_t)T * cldl, left);
+        A0[u] = Lb(oa0);
+        A1[u] = Lb(oa1);
+        B0[u] = Db(ob0);
+        B1[u] = Db(ob1);
       }
     };
     auto mfma = [&](int T0, const double *A0, const double *A1, const double *B0,
@@ -1513,7 +1547,7 @@ __device__ __forceinline__ int gather_tile(
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
           const int b = tb + u * (kThreads / 64);
-          if (b < ncol && kr >= kc0 + b) acc[mra][mc[kc0 - k0 + b]] += cv[u];
+          if (b < blim) acc[mra][mc[kc0 - k0 + b]] += (double)cv[u];
         }
       }
       for (int t0 = 0; t0 < K; t0 += 8 * KC) {
