@@ -336,6 +336,8 @@ struct Numeric {
   int64_t solve_ws_per_rhs = 0;           // doubles of workspace per right-hand side
   double *d_x = nullptr;
   size_t d_x_cap = 0;
+  double *d_b = nullptr;                  // right-hand sides of a refined host solve
+  size_t d_b_cap = 0;
   bool posdef = false;                    // A = L L^T (pivots in order, all > 0)
   spral_ssids_hip_stats stats{};
   double *d_aval = nullptr;               // copy of the factorized values
@@ -363,6 +365,7 @@ struct Numeric {
     if (d_bigtab) (void)hipFree(d_bigtab);
     if (d_X) (void)hipFree(d_X);
     if (d_x) (void)hipFree(d_x);
+    if (d_b) (void)hipFree(d_b);
     if (d_aval) (void)hipFree(d_aval);
     if (d_scal) (void)hipFree(d_scal);
     if (d_r) (void)hipFree(d_r);
@@ -1499,16 +1502,25 @@ static void solve_device(Numeric &N, int job, int nrhs, double *d_x, int ldx,
   solve_launch(N, job, nrhs, d_x, ldx, st, solve_ws(N, nrhs));
 }
 
+// A buffer of the handle, grown to need doubles and kept for the next call (a
+// hipFree waits for everything that runs on the device, other handles' work
+// included).
+static double *grown(double *&p, size_t &cap, size_t need) {
+  if (need > cap) {
+    if (p) HIPCHK(hipFree(p));
+    p = nullptr;
+    cap = 0;
+    HIPCHK(hipMalloc(&p, need * sizeof(double)));
+    cap = need;
+  }
+  return p;
+}
+
 static int solve_host(Numeric &N, int job, int nrhs, double *x, int ldx) {
   Symbolic &S = *N.symb;
   if (nrhs < 1 || ldx < S.n) return -10;
   HIPCHK(hipSetDevice(S.device));
-  size_t need = (size_t)S.n * nrhs;
-  if (need > N.d_x_cap) {
-    if (N.d_x) HIPCHK(hipFree(N.d_x));
-    HIPCHK(hipMalloc(&N.d_x, need * sizeof(double)));
-    N.d_x_cap = need;
-  }
+  grown(N.d_x, N.d_x_cap, (size_t)S.n * nrhs);
   HIPCHK(hipMemcpy2DAsync(N.d_x, S.n * sizeof(double), x, ldx * sizeof(double),
                           S.n * sizeof(double), nrhs, hipMemcpyHostToDevice, N.stream));
   solve_device(N, job, nrhs, N.d_x, S.n, N.stream);
@@ -2106,24 +2118,20 @@ int spral_ssids_hip_solve_refine(void *numeric, int nrhs, const double *b, doubl
   Numeric *N = static_cast<Numeric *>(numeric);
   const int n = N->symb->n;
   if (nrhs < 1 || ldx < n) return -10;
-  double *db = nullptr, *dx = nullptr;
-  int rc = 0;
   try {
     HIPCHK(hipSetDevice(N->symb->device));
-    HIPCHK(hipMalloc(&db, (size_t)n * nrhs * sizeof(double)));
-    HIPCHK(hipMalloc(&dx, (size_t)n * nrhs * sizeof(double)));
+    double *db = grown(N->d_b, N->d_b_cap, (size_t)n * nrhs);
+    double *dx = grown(N->d_x, N->d_x_cap, (size_t)n * nrhs);
     copy2d_now(db, n * sizeof(double), b, ldx * sizeof(double), n * sizeof(double),
                        nrhs, hipMemcpyHostToDevice, N->stream);
-    rc = refine_device(*N, nrhs, db, dx, n, maxit, tol, bwd, iters, N->stream);
+    const int rc = refine_device(*N, nrhs, db, dx, n, maxit, tol, bwd, iters, N->stream);
     HIPCHK(hipMemcpy2DAsync(x, ldx * sizeof(double), dx, n * sizeof(double),
                             n * sizeof(double), nrhs, hipMemcpyDeviceToHost, N->stream));
     HIPCHK(hipStreamSynchronize(N->stream));
+    return rc;
   } catch (HipError &) {
-    rc = -51;
+    return -51;
   }
-  if (db) (void)hipFree(db);
-  if (dx) (void)hipFree(dx);
-  return rc;
 }
 
 // Every front's D^{-1} (and, with pall, its eliminated variables), packed on
