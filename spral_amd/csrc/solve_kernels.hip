@@ -69,6 +69,14 @@ constexpr int kMrSplit = 4;
 // one instruction stream; each right-hand side keeps its own sequence)
 constexpr int kDiagGroup = 4;
 
+// A solution entry not yet published: a quiet NaN with a payload no operation
+// makes.  An entry that came out as these bits (an input NaN's payload carried
+// through) is published as another NaN.
+constexpr unsigned long long kUnset = 0x7ff85e7b19c3d24aull;
+__device__ inline bool is_unset(double v) {
+  return (unsigned long long)__double_as_longlong(v) == kUnset;
+}
+
 // value of v in lane j (j uniform)
 __device__ inline double bcast_lane(double v, int j) {
   const long long b = __double_as_longlong(v);
@@ -239,6 +247,9 @@ __global__ __launch_bounds__(kThreads) void k_fwd_tri(const SolveNode *sn, const
         __syncthreads();
       }
       for (int p = tid; p < ne; p += kThreads) xr[Pperm[p]] = acc[p];
+    } else {  // the triangle's solution is published there (k_big_fwd_lvl)
+      double *Y = solve_P(ws, P, nrhs) + (size_t)r * ne;
+      for (int p = tid; p < ne; p += kThreads) Y[p] = __longlong_as_double((long long)kUnset);
     }
     if (acc != (double *)X)
       for (int p = tid; p < n; p += kThreads) X[p] = acc[p];
@@ -540,7 +551,12 @@ __global__ __launch_bounds__(kThreads) void k_bwd_tri(const SolveNode *sn, const
                  (((pr[0][tid] + pr[1][tid]) + pr[2][tid]) + pr[3][tid]);
       __syncthreads();
     }
-    if (ne > kBigTri) continue;  // the triangle is solved by the big-front launches
+    if (ne > kBigTri) {  // the triangle is solved by k_big_bwd_lvl, published there
+      // (this right-hand side's first partial sums, all read by now)
+      double *Y = solve_P(ws, P, nrhs) + (size_t)r * ne;
+      for (int j = tid; j < ne; j += kThreads) Y[j] = __longlong_as_double((long long)kUnset);
+      continue;
+    }
     for (int b = idiv_up(ne, kBlk) - 1; b >= 0; --b) {
       const int j0 = b * kBlk, j1 = imin(j0 + kBlk, ne), wb = j1 - j0, rows = ne - j1;
       stage_lower(PL, ldl, j0, wb, lb);
@@ -574,32 +590,46 @@ __global__ __launch_bounds__(kThreads) void k_bwd_tri(const SolveNode *sn, const
 // ---- big fronts: one launch per tree level ---------------------------------
 // Fronts with ne > kBigTri solve their triangle, L11 y = X[0:ne] (forward) or
 // L11^T x = X[0:ne] (backward), in one launch per tree level over 64-column
-// blocks: a workgroup per block of every big front of the level.  Within a
-// front, workgroups take their blocks by ticket (an atomic counter; forward
-// in increasing, backward in decreasing block order), so a workgroup waits
-// only for blocks whose workgroups took their tickets earlier and are
+// blocks: a workgroup per block of every big front of the level and per group
+// of 16 right-hand sides (gridDim.y groups, up to kBigGroups).  Within a
+// front and group, workgroups take their blocks by ticket (an atomic counter;
+// forward in increasing, backward in decreasing block order), so a workgroup
+// waits only for blocks whose workgroups took their tickets earlier and are
 // running: every wait ends.  Block b's workgroup accumulates the products of
-// the blocks it depends on in block order (not arrival order), solves its
-// diagonal block on one wave per right-hand side, stores the block's
-// solution into X and x, and raises the block's flag.  The flag is a
-// device-scope release store after a workgroup barrier; readers poll it with
-// relaxed device-scope loads and read the published solutions with
-// device-scope loads (coherent across the XCDs' L2 caches).  The sync words
-// (per big front: forward ticket and one flag per block, then the same for
-// the backward solve) live after the call's workspace and are cleared by
-// k_big_sync_clear at the start of every solve.
+// the blocks it depends on in block order (not arrival order) and solves its
+// diagonal block, right-hand sides dealt to the waves.
+// The chain of blocks bounds it: what a hop costs is the time from one block's
+// solution to the next one's.  A block's solution is its own flag: the front's
+// part of P (unused while the triangle is solved) is set to kUnset by the
+// launch before, the solution is stored there with device-scope stores, and
+// the readers load the values themselves until none is kUnset.  With a flag of
+// its own a block put a release (a write-back of the XCD's L2) and a second
+// round trip into every hop: on a 4,160-column root with one right-hand side
+// a hop took 5.3 us and takes 2.95; on a 2,350-column root with 64, all in
+// one group, it took 27 us and takes 6.5 in four groups.
+// The tickets (per big front nb + 1 words for the forward solve, of which the
+// first kBigGroups are used, then as many for the backward solve; nb > 4)
+// live after the call's workspace and are cleared by k_big_sync_clear at the
+// start of every solve.
+constexpr int kBigGroups = 4;
 __device__ inline double load_dev(const double *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline void wait_flag(const int *f) {
-  while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-    __builtin_amdgcn_s_sleep(1);
-  // the solution loads that follow stay behind the poll (a compiler barrier;
-  // the hardware issues them only after the poll's value has returned)
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+__device__ inline void publish(double *p, double v) {
+  if (is_unset(v)) v = __longlong_as_double((long long)(kUnset ^ 1));
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline void raise_flag(int *f) {
-  __hip_atomic_store(f, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+// v[u] = y[off(u)], once every lane's 16 entries are published
+template <class Off>
+__device__ inline void wait_values(const double *y, Off off, double (&v)[16]) {
+  bool miss;
+  do {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = load_dev(y + off(u));
+    miss = false;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) miss |= is_unset(v[u]);
+  } while (__ballot(miss) != 0);
 }
 
 __global__ void k_big_sync_clear(int *sync, int n) {
@@ -608,38 +638,92 @@ __global__ void k_big_sync_clear(int *sync, int n) {
 }
 
 // The products of the other blocks go to FP64 MFMA (v_mfma_f64_16x16x4f64)
-// for up to 64 right-hand sides at once: wave w takes 16 rows (forward) or
+// for a group of up to 16 right-hand sides: wave w takes 16 rows (forward) or
 // 16 columns (backward) of block b, the right-hand sides are the 16-wide
 // output columns, and the 64 positions of each other block are the K
 // dimension in steps of 4, in block order.  An output column depends only
 // on its own right-hand side, so every column is the same whatever nrhs.
 // The diagonal block is then solved once per right-hand side (lane = row,
-// the right-hand sides dealt to the waves in turn).
+// the right-hand sides dealt to the waves in turn).  The next block's part of
+// L is loaded before the wait for the current one.
+
+// L of one wave's 16 outputs against the 64 positions of a block, and the
+// accumulation of a block's product
+__device__ inline void big_mfma(const double (&av)[16], const double (&bv)[16], bool on,
+                                mr_acc_t (&acc)[kMrSplit]) {
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    acc[u % kMrSplit] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], on ? bv[u] : 0.0,
+                                                             acc[u % kMrSplit], 0, 0, 0);
+}
+
+// The diagonal block for the group's right-hand sides, G to a wave: lane i
+// starts from its initial value x0 minus the products' sum (red) and takes
+// part j of the substitution (in ascending order forward, descending backward)
+// from lane j; l[j] is lane i's factor for part j.  Published to Y, kept in X
+// and x.
+template <bool FWD, int G>
+__device__ inline void big_diag(const double (&l)[kBlk], const double (*red)[kBlk],
+                                const double (&x0)[kDiagGroup], double *X, size_t m, double *Y,
+                                size_t ldy, double *x, size_t ldx, int var, int j0, int wb,
+                                int nr, int lane, int wave) {
+  double v[G];
+#pragma unroll
+  for (int r = 0; r < G; ++r) v[r] = (lane < wb) ? x0[r] - red[wave * G + r][lane] : 0.0;
+#pragma unroll
+  for (int jj = 0; jj < kBlk; ++jj) {
+    const int j = FWD ? jj : kBlk - 1 - jj;
+#pragma unroll
+    for (int r = 0; r < G; ++r) v[r] = fma(-l[j], bcast_lane(v[r], j), v[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < G; ++r) {
+    const int q = wave * G + r;
+    if (q < nr && lane < wb) publish(Y + (size_t)q * ldy + j0 + lane, v[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < G; ++r) {
+    const int q = wave * G + r;
+    if (q < nr && lane < wb) {
+      X[(size_t)q * m + j0 + lane] = v[r];
+      x[(size_t)q * ldx + var] = v[r];
+    }
+  }
+}
+// right-hand sides a wave takes in a group of nr (16 / kGroups = kDiagGroup)
+static_assert(kDiagGroup * kGroups == 16, "a group's right-hand sides, once over the waves");
+__device__ inline void big_x0(const double *X, size_t m, int j0, int wb, int nr, int lane,
+                              int wave, double (&x0)[kDiagGroup]) {
+  const int G = (nr > kGroups) ? kDiagGroup : 1;
+#pragma unroll
+  for (int r = 0; r < kDiagGroup; ++r)
+    x0[r] = masked(X[(size_t)imin(wave * G + r, nr - 1) * m + j0 + imin(lane, wb - 1)],
+                   r < G && wave * G + r < nr);
+}
 
 // forward: block b's rows minus L[b rows, earlier columns] Y[earlier]
 __global__ __launch_bounds__(kThreads) void k_big_fwd_lvl(const SolveNode *sn, const int *boff,
                                                           const int *bslot, const int *bsync,
                                                           int nbig, double *x, int ldx,
                                                           int nrhs, double *ws, int *sync) {
-  __shared__ double red[16 * kMrChunks][kBlk];
+  __shared__ double red[16][kBlk];
   __shared__ int s_b;
   const int li = table_find(boff, nbig, blockIdx.x);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
-  int *tick = sync + bsync[li];
-  int *flag = tick + 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ri = lane & 15, kq = lane >> 4;
-  if (tid == 0) s_b = atomicAdd(tick, 1);
+  if (tid == 0) s_b = atomicAdd(sync + bsync[li] + blockIdx.y, 1);
   __syncthreads();
   const int b = s_b;
   gcdouble *PL = (gcdouble *)P.L;
   gcint *Pperm = (gcint *)P.perm;
-  double *PX = solve_X(ws, P, nrhs);
+  double *PX = solve_X(ws, P, nrhs), *PY = solve_P(ws, P, nrhs);
   const int ldl = P.ldl, m = P.m, ne = P.nelim;
   const int j0 = b * kBlk, j1 = imin(j0 + kBlk, ne), wb = j1 - j0;
+  const int var = Pperm[j0 + imin(lane, wb - 1)];
   // A operand row of this lane (the wave's 16 rows of block b, clamped)
-  const int arow = j0 + imin(16 * wave + ri, wb - 1);
+  gcdouble *La = PL + j0 + imin(16 * wave + ri, wb - 1);
   // L of the diagonal block for the substitutions (lane = row), loaded once
   double l[kBlk];
   {
@@ -648,69 +732,43 @@ __global__ __launch_bounds__(kThreads) void k_big_fwd_lvl(const SolveNode *sn, c
     for (int j = 0; j < kBlk; ++j)
       l[j] = masked(PL[(size_t)(j0 + imin(j, wb - 1)) * ldl + rr], j < lane && lane < wb);
   }
-  for (int rc = 0; rc < nrhs; rc += 16 * kMrChunks) {
-    const int nr = imin(16 * kMrChunks, nrhs - rc);
-    mr_acc_t acc[kMrChunks][kMrSplit];
+  for (int rc = 16 * blockIdx.y; rc < nrhs; rc += 16 * gridDim.y) {
+    const int nr = imin(16, nrhs - rc);
+    double *X = PX + (size_t)rc * m, *Y = PY + (size_t)rc * ne;
+    const double *y = Y + (size_t)imin(ri, nr - 1) * ne + kq;
+    double x0[kDiagGroup];
+    big_x0(X, m, j0, wb, nr, lane, wave, x0);
+    mr_acc_t acc[kMrSplit];
 #pragma unroll
-    for (int h = 0; h < kMrChunks; ++h)
+    for (int t = 0; t < kMrSplit; ++t) acc[t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
+    double av[16];
+    // every block before b is a full block
 #pragma unroll
-      for (int t = 0; t < kMrSplit; ++t) acc[h][t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
-    for (int j = 0; j < b; ++j) {  // every block before b is a full block
-      const int c0 = j * kBlk;
-      double av[16];
+    for (int u = 0; u < 16; ++u) av[u] = La[(size_t)(b > 0 ? 4 * u + kq : 0) * ldl];
+    for (int j = 0; j < b; ++j) {
+      const int cn = imin(j + 1, b - 1) * kBlk;
+      double an[16], bv[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) av[u] = PL[(size_t)(c0 + 4 * u + kq) * ldl + arow];
-      if (rc == 0) wait_flag(flag + j);
+      for (int u = 0; u < 16; ++u) an[u] = La[(size_t)(cn + 4 * u + kq) * ldl];
+      wait_values(y + j * kBlk, [](int u) { return 4 * u; }, bv);
+      big_mfma(av, bv, ri < nr, acc);
 #pragma unroll
-      for (int h = 0; h < kMrChunks; ++h) {
-        if (16 * h >= nr) break;
-        const int q = 16 * h + ri;
-        const double *y = PX + (size_t)(rc + imin(q, nr - 1)) * m + c0 + kq;
-        double bv[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) bv[u] = masked(load_dev(y + 4 * u), q < nr);
-#pragma unroll
-        for (int u = 0; u < 16; ++u)
-          acc[h][u % kMrSplit] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              av[u], bv[u], acc[h][u % kMrSplit], 0, 0, 0);
-      }
+      for (int u = 0; u < 16; ++u) av[u] = an[u];
     }
-    // element (row kq + 4 rg of the wave's rows, right-hand side ri) of chunk h
+    // element (row kq + 4 rg of the wave's rows, right-hand side ri)
 #pragma unroll
-    for (int h = 0; h < kMrChunks; ++h)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg)
-        red[16 * h + ri][16 * wave + kq + 4 * rg] =
-            ((acc[h][0][rg] + acc[h][1][rg]) + acc[h][2][rg]) + acc[h][3][rg];
+    for (int rg = 0; rg < 4; ++rg)
+      red[ri][16 * wave + kq + 4 * rg] =
+          ((acc[0][rg] + acc[1][rg]) + acc[2][rg]) + acc[3][rg];
     __syncthreads();
-    auto diag = [&](auto grp) {
-      constexpr int G = decltype(grp)::value;
-      for (int q0 = wave * G; q0 < nr; q0 += kGroups * G) {
-        double v[G];
-#pragma unroll
-        for (int r = 0; r < G; ++r) {
-          const int q = q0 + r;
-          v[r] = (q < nr && lane < wb) ? PX[(size_t)(rc + q) * m + j0 + lane] - red[q][lane] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kBlk; ++j)
-#pragma unroll
-          for (int r = 0; r < G; ++r) v[r] = fma(-l[j], bcast_lane(v[r], j), v[r]);
-#pragma unroll
-        for (int r = 0; r < G; ++r) {
-          const int q = q0 + r;
-          if (q < nr && lane < wb) {
-            PX[(size_t)(rc + q) * m + j0 + lane] = v[r];
-            x[(size_t)(rc + q) * ldx + Pperm[j0 + lane]] = v[r];
-          }
-        }
-      }
-    };
-    if (nr > kGroups) diag(std::integral_constant<int, kDiagGroup>());
-    else diag(std::integral_constant<int, 1>());
+    if (nr > kGroups)
+      big_diag<true, kDiagGroup>(l, red, x0, X, m, Y, ne, x + (size_t)rc * ldx, ldx, var, j0,
+                                  wb, nr, lane, wave);
+    else if (wave < nr)
+      big_diag<true, 1>(l, red, x0, X, m, Y, ne, x + (size_t)rc * ldx, ldx, var, j0, wb, nr,
+                         lane, wave);
     __syncthreads();
   }
-  if (tid == 0) raise_flag(flag + b);
 }
 
 // backward: block b's values minus L[later rows, b columns]^T X[later]
@@ -719,96 +777,75 @@ __global__ __launch_bounds__(kThreads) void k_big_bwd_lvl(const SolveNode *sn, c
                                                           int nbig, double *x, int ldx,
                                                           int nrhs, double *ws, int *sync) {
   __shared__ double lb[kBlk][kBlk + 1];
-  __shared__ double red[16 * kMrChunks][kBlk];
+  __shared__ double red[16][kBlk];
   __shared__ int s_b;
   const int li = table_find(boff, nbig, blockIdx.x);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
   const int ne = P.nelim, nb = idiv_up(ne, kBlk);
-  int *tick = sync + bsync[li] + nb + 1;
-  int *flag = tick + 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ri = lane & 15, kq = lane >> 4;
-  if (tid == 0) s_b = nb - 1 - atomicAdd(tick, 1);
+  if (tid == 0) s_b = nb - 1 - atomicAdd(sync + bsync[li] + nb + 1 + blockIdx.y, 1);
   __syncthreads();
   const int b = s_b;
   gcdouble *PL = (gcdouble *)P.L;
   gcint *Pperm = (gcint *)P.perm;
-  double *PX = solve_X(ws, P, nrhs);
+  double *PX = solve_X(ws, P, nrhs), *PY = solve_P(ws, P, nrhs);
   const int ldl = P.ldl, m = P.m;
   const int j0 = b * kBlk, j1 = imin(j0 + kBlk, ne), wb = j1 - j0;
+  const int var = Pperm[j0 + imin(lane, wb - 1)];
   stage_lower(PL, ldl, j0, wb, lb);
+  __syncthreads();
+  double c[kBlk];
+#pragma unroll
+  for (int i = 0; i < kBlk; ++i) c[i] = lb[i][lane];
   // A operand column of this lane (the wave's 16 columns of block b, clamped)
-  const int acol = j0 + imin(16 * wave + ri, wb - 1);
-  for (int rc = 0; rc < nrhs; rc += 16 * kMrChunks) {
-    const int nr = imin(16 * kMrChunks, nrhs - rc);
-    mr_acc_t acc[kMrChunks][kMrSplit];
+  gcdouble *La = PL + (size_t)(j0 + imin(16 * wave + ri, wb - 1)) * ldl;
+  auto load_a = [&](int j, double (&a)[16]) {
+    const int r0 = j * kBlk, rows = imin(kBlk, ne - r0);
 #pragma unroll
-    for (int h = 0; h < kMrChunks; ++h)
+    for (int u = 0; u < 16; ++u)
+      a[u] = masked(La[r0 + imin(4 * u + kq, rows - 1)], 4 * u + kq < rows);
+  };
+  for (int rc = 16 * blockIdx.y; rc < nrhs; rc += 16 * gridDim.y) {
+    const int nr = imin(16, nrhs - rc);
+    double *X = PX + (size_t)rc * m, *Y = PY + (size_t)rc * ne;
+    const double *y = Y + (size_t)imin(ri, nr - 1) * ne;
+    double x0[kDiagGroup];
+    big_x0(X, m, j0, wb, nr, lane, wave, x0);
+    mr_acc_t acc[kMrSplit];
 #pragma unroll
-      for (int t = 0; t < kMrSplit; ++t) acc[h][t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
+    for (int t = 0; t < kMrSplit; ++t) acc[t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
+    double av[16];
+    load_a(nb - 1, av);
     for (int j = nb - 1; j > b; --j) {
       const int r0 = j * kBlk, rows = imin(kBlk, ne - r0);
-      double av[16];
+      double an[16], bv[16];
+      load_a(imax(j - 1, b + 1), an);
+      wait_values(y + r0, [&](int u) { return imin(4 * u + kq, rows - 1); }, bv);
+      // (rows past the last block's end: zero in av, and 0 * NaN is avoided)
+      if (rows < kBlk) {
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-        av[u] = masked(PL[(size_t)acol * ldl + r0 + imin(4 * u + kq, rows - 1)],
-                       4 * u + kq < rows);
-      if (rc == 0) wait_flag(flag + j);
-#pragma unroll
-      for (int h = 0; h < kMrChunks; ++h) {
-        if (16 * h >= nr) break;
-        const int q = 16 * h + ri;
-        const double *xq = PX + (size_t)(rc + imin(q, nr - 1)) * m + r0;
-        double bv[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u)
-          bv[u] = masked(load_dev(xq + imin(4 * u + kq, rows - 1)), q < nr && 4 * u + kq < rows);
-#pragma unroll
-        for (int u = 0; u < 16; ++u)
-          acc[h][u % kMrSplit] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              av[u], bv[u], acc[h][u % kMrSplit], 0, 0, 0);
+        for (int u = 0; u < 16; ++u) bv[u] = masked(bv[u], 4 * u + kq < rows);
       }
+      big_mfma(av, bv, ri < nr, acc);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) av[u] = an[u];
     }
-    // element (column kq + 4 rg of the wave's columns, right-hand side ri)
+    // element (row kq + 4 rg of the wave's columns, right-hand side ri)
 #pragma unroll
-    for (int h = 0; h < kMrChunks; ++h)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg)
-        red[16 * h + ri][16 * wave + kq + 4 * rg] =
-            ((acc[h][0][rg] + acc[h][1][rg]) + acc[h][2][rg]) + acc[h][3][rg];
+    for (int rg = 0; rg < 4; ++rg)
+      red[ri][16 * wave + kq + 4 * rg] =
+          ((acc[0][rg] + acc[1][rg]) + acc[2][rg]) + acc[3][rg];
     __syncthreads();
-    double c[kBlk];
-#pragma unroll
-    for (int i = 0; i < kBlk; ++i) c[i] = lb[i][lane];
-    auto diag = [&](auto grp) {
-      constexpr int G = decltype(grp)::value;
-      for (int q0 = wave * G; q0 < nr; q0 += kGroups * G) {
-        double v[G];
-#pragma unroll
-        for (int r = 0; r < G; ++r) {
-          const int q = q0 + r;
-          v[r] = (q < nr && lane < wb) ? PX[(size_t)(rc + q) * m + j0 + lane] - red[q][lane] : 0.0;
-        }
-#pragma unroll
-        for (int i = kBlk - 1; i >= 0; --i)
-#pragma unroll
-          for (int r = 0; r < G; ++r) v[r] = fma(-c[i], bcast_lane(v[r], i), v[r]);
-#pragma unroll
-        for (int r = 0; r < G; ++r) {
-          const int q = q0 + r;
-          if (q < nr && lane < wb) {
-            PX[(size_t)(rc + q) * m + j0 + lane] = v[r];
-            x[(size_t)(rc + q) * ldx + Pperm[j0 + lane]] = v[r];
-          }
-        }
-      }
-    };
-    if (nr > kGroups) diag(std::integral_constant<int, kDiagGroup>());
-    else diag(std::integral_constant<int, 1>());
+    if (nr > kGroups)
+      big_diag<false, kDiagGroup>(c, red, x0, X, m, Y, ne, x + (size_t)rc * ldx, ldx, var, j0,
+                                  wb, nr, lane, wave);
+    else if (wave < nr)
+      big_diag<false, 1>(c, red, x0, X, m, Y, ne, x + (size_t)rc * ldx, ldx, var, j0, wb, nr,
+                         lane, wave);
     __syncthreads();
   }
-  if (tid == 0) raise_flag(flag + b);
 }
 
 // ---- launchers ----------------------------------------------------------------
@@ -822,13 +859,13 @@ int bwd_cols_per_wg() { return kBwdCols; }
 void launch_big_fwd_lvl(hipStream_t st, const SolveNode *sn, const int *tab, int nbig, int nwg,
                         double *x, int ldx, int nrhs, double *ws, int *sync) {
   if (nbig <= 0) return;
-  hipLaunchKernelGGL(k_big_fwd_lvl, dim3(nwg), dim3(kThreads), 0, st, sn, tab, tab + nbig + 1,
+  hipLaunchKernelGGL(k_big_fwd_lvl, dim3(nwg, imin(idiv_up(nrhs, 16), kBigGroups)), dim3(kThreads), 0, st, sn, tab, tab + nbig + 1,
                      tab + 2 * nbig + 1, nbig, x, ldx, nrhs, ws, sync);
 }
 void launch_big_bwd_lvl(hipStream_t st, const SolveNode *sn, const int *tab, int nbig, int nwg,
                         double *x, int ldx, int nrhs, double *ws, int *sync) {
   if (nbig <= 0) return;
-  hipLaunchKernelGGL(k_big_bwd_lvl, dim3(nwg), dim3(kThreads), 0, st, sn, tab, tab + nbig + 1,
+  hipLaunchKernelGGL(k_big_bwd_lvl, dim3(nwg, imin(idiv_up(nrhs, 16), kBigGroups)), dim3(kThreads), 0, st, sn, tab, tab + nbig + 1,
                      tab + 2 * nbig + 1, nbig, x, ldx, nrhs, ws, sync);
 }
 void launch_big_sync_clear(hipStream_t st, int *sync, int n) {
