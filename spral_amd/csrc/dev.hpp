@@ -174,6 +174,32 @@ __device__ inline double masked(double v, bool keep) {
   return keep ? v : 0.0;
 }
 
+// Guarded loads without branches: a buffer load whose byte offset is at or
+// past the buffer's length reads nothing and returns zero, so a lane that has
+// nothing to load takes the offset kNoLoad.  (As conditional expressions the
+// same loads became branches, and those of FP32 blocks waited for each value
+// in turn to convert it: 12 us of a tile's 30.)  The base and the length are
+// uniform; lengths stay below 2^31.
+constexpr unsigned kNoLoad = 0xfffffff0u;
+typedef unsigned uint2v_t __attribute__((ext_vector_type(2)));
+template <typename T>
+struct LoadBuffer {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ LoadBuffer(const T *base, int64_t bytes)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T *>(base), 0,
+            (int)(bytes < 0 ? 0 : bytes > 0x7fffffff ? 0x7fffffff : bytes), 0x00020000)) {}
+  // soff: a uniform part of the offset (not together with kNoLoad)
+  __device__ T operator()(unsigned off, unsigned soff = 0) const {
+    if constexpr (sizeof(T) == 4) {
+      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off, soff, 0));
+    } else {
+      const uint2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, soff, 0);
+      return __hiloint2double((int)v.y, (int)v.x);
+    }
+  }
+};
+
 // value held by lane 0 (wave-uniform by construction), as a scalar
 __device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ inline double uni(double v) {
@@ -181,6 +207,14 @@ __device__ inline double uni(double v) {
   const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
   const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// v, recomputed from here on: what depends on it is not kept in registers
+// across the iterations of a loop around
+__device__ inline int fresh(int v) {
+  v = uni(v);
+  asm volatile("" : "+s"(v));
+  return v;
 }
 
 // Wave-wide maxima with DPP lane permutations inside each row of 16 lanes

@@ -1317,31 +1317,6 @@ __global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, const int *
   }
 }
 
-// Guarded loads without branches: a buffer load whose byte offset is at or
-// past the buffer's length reads nothing and returns zero, so a lane that has
-// nothing to load takes the offset kNoLoad.  (As conditional expressions the
-// same loads became branches, and those of FP32 blocks waited for each value
-// in turn to convert it: 12 us of a tile's 30.)  The base and the length are
-// uniform; lengths stay below 2^31.
-constexpr unsigned kNoLoad = 0xfffffff0u;
-typedef unsigned uint2v_t __attribute__((ext_vector_type(2)));
-template <typename T>
-struct LoadBuffer {
-  __amdgpu_buffer_rsrc_t rsrc;
-  __device__ LoadBuffer(const T *base, int64_t bytes)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T *>(base), 0,
-            (int)(bytes < 0 ? 0 : bytes > 0x7fffffff ? 0x7fffffff : bytes), 0x00020000)) {}
-  __device__ T operator()(unsigned off) const {
-    if constexpr (sizeof(T) == 4) {
-      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
-    } else {
-      const uint2v_t v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0);
-      return __hiloint2double((int)v.y, (int)v.x);
-    }
-  }
-};
-
 // PART 0: every tile of the level's fronts; 1: the first tile column only
 // (the pivot block and the rows below it); 2: the remaining tiles
 // Returns the front's slot when this workgroup built the front's first

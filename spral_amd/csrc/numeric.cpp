@@ -52,10 +52,10 @@ void launch_fwd_tri(hipStream_t, int, const SolveNode *, const int *, const int 
                     int, int, double *);
 void launch_fwd_rows(hipStream_t, int, const SolveNode *, const int *, const int *, int,
                      const int *, int, double *);
-void launch_big_fwd_lvl(hipStream_t, const SolveNode *, const int *, int, int, double *, int,
-                        int, double *, int *);
+void launch_big_fwd_lvl(hipStream_t, const SolveNode *, const int *, int, int, const int *,
+                        double *, int, int, double *, int *);
 void launch_big_bwd_lvl(hipStream_t, const SolveNode *, const int *, int, int, double *, int,
-                        int, double *, int *);
+                        int, double *, int *, int);
 void launch_big_sync_clear(hipStream_t, int *, int);
 int big_tri_threshold();
 int fwd_rows_per_wg();
@@ -63,7 +63,7 @@ int bwd_rows_per_wg();
 int bwd_cols_per_wg();
 void launch_dsolve(hipStream_t, int, const SolveNode *, double *, int, int, int);
 void launch_bwd(hipStream_t, int, const SolveNode *, const int *, double *, int, int,
-                const int *, const int *, int, double *, int);
+                const int *, const int *, int, double *, int, int);
 
 void launch_residual(hipStream_t, int, const int64_t *, const int *, const int64_t *,
                      const double *, const double *, const double *, double *, int, int);
@@ -1449,10 +1449,11 @@ static void solve_launch(Numeric &N, int job, int nrhs, double *d_x, int ldx, hi
   if (fwd || bwd) launch_big_sync_clear(st, sync, (int)N.solve_sync_ints);
   if (fwd)
     for (int L = 0; L < nlev; ++L) {
-      const int nl = S.lvl_ptr[L + 1] - S.lvl_ptr[L];
-      launch_fwd_tri(st, nl, N.d_sn, slots + S.lvl_ptr[L], S.d_child, d_x, ldx, nrhs, ws);
-      launch_big_fwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], (int)N.big_of_level[L].size(),
-                         N.big_blocks[L], d_x, ldx, nrhs, ws, sync);
+      const int nl = S.lvl_ptr[L + 1] - S.lvl_ptr[L], nbig = (int)N.big_of_level[L].size();
+      if (nl > nbig)
+        launch_fwd_tri(st, nl, N.d_sn, slots + S.lvl_ptr[L], S.d_child, d_x, ldx, nrhs, ws);
+      launch_big_fwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], nbig, N.big_blocks[L],
+                         S.d_child, d_x, ldx, nrhs, ws, sync);
       launch_fwd_rows(st, nl, N.d_sn, slots + S.lvl_ptr[L], S.d_child, nrhs,
                       N.d_gemv_tab + N.gemv_tab_off[L], N.gemv_total[L], ws);
     }
@@ -1464,11 +1465,12 @@ static void solve_launch(Numeric &N, int job, int nrhs, double *d_x, int ldx, hi
     launch_dsolve(st, S.nnodes, N.d_sn, d_x, ldx, nrhs, 1);
   if (bwd)
     for (int L = nlev - 1; L >= 0; --L) {
-      launch_bwd(st, S.lvl_ptr[L + 1] - S.lvl_ptr[L], N.d_sn, slots + S.lvl_ptr[L], d_x,
-                 ldx, nrhs, N.d_gemv_tab + N.bwd_tab_off[L], N.d_gemv_tab + N.bwdc_tab_off[L],
-                 N.bwdc_total[L], ws, dfuse);
-      launch_big_bwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], (int)N.big_of_level[L].size(),
-                         N.big_blocks[L], d_x, ldx, nrhs, ws, sync);
+      const int nl = S.lvl_ptr[L + 1] - S.lvl_ptr[L], nbig = (int)N.big_of_level[L].size();
+      launch_bwd(st, nl, N.d_sn, slots + S.lvl_ptr[L], d_x, ldx, nrhs,
+                 N.d_gemv_tab + N.bwd_tab_off[L], N.d_gemv_tab + N.bwdc_tab_off[L],
+                 N.bwdc_total[L], ws, dfuse, nl - nbig);
+      launch_big_bwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], nbig, N.big_blocks[L], d_x,
+                         ldx, nrhs, ws, sync, dfuse);
     }
   HIPCHK(hipGetLastError());
 }

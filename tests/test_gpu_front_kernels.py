@@ -54,3 +54,39 @@ def test_big_front_groups(lib, n, nrhs):
     keep = [k for k in range(nrhs) if k not in (1, 2)]
     assert np.array_equal(y[:, keep], x[:, keep])
     ssids.ssids_free(ak, fk)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130, 256])
+def test_front_groups(lib, n):
+    """Triangles of up to 256 columns: one right-hand side, groups of four and
+    of 16 give the same columns bit for bit."""
+    m = dense_lower(block(n, "dominant"))
+    ak, fk, _, opts = gpu_factor(m)
+    _, b = rhs(m, 2100, 7)
+    ref = np.stack([gpu_solve(ak, fk, opts, b[:, k]) for k in range(17)], axis=1)
+    assert matrices.bwd_error(m.full, ref, b[:, :17]).max() <= RAW_TOL
+    for nrhs in (2, 4, 5, 16, 17, 2100):    # past 2,048 one front's groups are of 16
+        x = gpu_solve(ak, fk, opts, b[:, :nrhs])
+        k = min(nrhs, 17)
+        assert np.array_equal(x[:, :k], ref[:, :k]), nrhs
+        if nrhs == 2100:
+            assert matrices.bwd_error(m.full, x, b).max() <= RAW_TOL
+    ssids.ssids_free(ak, fk)
+
+
+@pytest.mark.parametrize("nrhs", [2, 5, 33])
+def test_grid_groups(lib, nrhs):
+    """A 14 x 13 x 11 stencil and a KKT system with delayed pivots (columns
+    between the eliminated ones and the rows): every level's kernels, whole and
+    ragged row blocks, against single-right-hand-side solves and jobs."""
+    for m in (matrices.laplace3d(14, 13, 11, diag=5.7), matrices.kkt_laplace(grid=8, m_con=100)):
+        ak, fk, _, opts = gpu_factor(m)
+        _, b = rhs(m, nrhs, 8)
+        x = gpu_solve(ak, fk, opts, b)
+        assert matrices.bwd_error(m.full, x, b).max() <= RAW_TOL
+        for k in (0, nrhs - 1):
+            assert np.array_equal(gpu_solve(ak, fk, opts, b[:, k]), x[:, k]), k
+        y = gpu_solve(ak, fk, opts, b, job=ssids.SSIDS_SOLVE_JOB_FWD)
+        y = gpu_solve(ak, fk, opts, y, job=ssids.SSIDS_SOLVE_JOB_DIAG_BWD)
+        assert np.allclose(y, x, rtol=1e-12, atol=1e-12)
+        ssids.ssids_free(ak, fk)
