@@ -16,9 +16,8 @@
 //               land on the rows (summed in LDS in a fixed order) minus
 //               L[rows, 0:ne] X[0:ne].  X[ne:m] is what the parent gathers.
 // Backward (root -> leaves), two launches per level:
-//   k_bwd_rows_mr: 256-row workgroups over [ne, m) write partial sums of
-//               L[rows, 0:ne]^T x[rows] (FP64 MFMA, up to 64 right-hand sides
-//               a pass);
+//   k_bwd_rows: 256-row workgroups over [ne, m) write partial sums of
+//               L[rows, 0:ne]^T x[rows];
 //   k_bwd_tri : a workgroup per front (ne <= kBigTri) and group of right-hand
 //               sides: the partials reduced in workgroup order, then the
 //               triangle with L11^T.
@@ -59,7 +58,6 @@ __device__ inline int find_node_s(const int *wg_off, int nlvl, int b) {
 
 // FP64 MFMA accumulators of the multi-right-hand-side products
 typedef double mr_acc_t __attribute__((ext_vector_type(4)));
-constexpr int kMrChunks = 4;  // 16-column MFMA outputs per wave: 64 right-hand sides a pass
 // independent accumulators per output (4-position step u goes to u % kMrSplit,
 // the partial sums added in order at the end): 16 dependent MFMAs become
 // 4 chains of 4
@@ -526,33 +524,32 @@ __global__ void k_dsolve(const SolveNode *sn, int nslots, double *x, int ldx, in
 
 // ---- backward -------------------------------------------------------------
 // Workgroups over 256-row blocks of [ne, m) times kBwdCols-column chunks of
-// [0, ne), for every front of the level (a row per thread):
+// [0, ne), for every front of the level:
 // part[rb][r][j] = sum over row block rb's rows i of L[i, j] x[var(i), r].
-// Columns go 16 at a time: the wave's 64 row products are summed by a
-// reduce-scatter, then the four waves' sums in wave order.  Each (rb, j) is
-// written by exactly one workgroup, so the sums do not depend on the split.
+// Each (rb, j) is written by exactly one workgroup, so the sums do not depend
+// on the split.
+// On FP64 MFMA for any number of right-hand sides (one kernel for every nrhs,
+// so each column is the same whatever nrhs): wave w takes rows 64w..64w+63 for
+// the 64 columns (four outputs of 16 columns by 16 right-hand sides, so a
+// value of x serves four products) and the waves' sums are added in wave
+// order.  Of the wave's rows lane quarter kq takes 16 kq..16 kq + 15, one a
+// step, so a lane's loads of a column are 128 contiguous bytes; all of a
+// wave's part of L is on its way before the variables of its rows are known.
+// With a wave per 16 columns, stepping through the 256 rows in eight batches,
+// each batch waited for its x: 19 us where 17 workgroups run (now 14), and
+// with 64 right-hand sides 103 us for a level of 510 (now 75).
 constexpr int kBwdCols = 64;
-
-// k_bwd_rows on FP64 MFMA for any number of right-hand sides (the launch
-// used for every nrhs, so each column is the same whatever nrhs): wave w
-// takes columns 16w..16w+15 of the workgroup's 64-column chunk, the
-// right-hand sides are the 16-wide output columns (64 a pass), and the
-// workgroup's 256 rows the K dimension in steps of 4, in row order, dealt to
-// kMrSplit accumulators whose sums are added in order.
-// NCH: 16-column output chunks per pass (1 for up to 16 right-hand sides,
-// which keeps the registers for several workgroups per CU; a column's
-// arithmetic is the same in both instantiations)
-template <int NCH>
-__global__ __launch_bounds__(kThreads) void k_bwd_rows_mr(const SolveNode *sn, const int *slots,
-                                                          const int *wg_off, int nlvl,
-                                                          const double *x, int ldx, int nrhs,
-                                                          double *ws) {
-  constexpr int kSteps = 8;  // 4-row steps loaded per batch
-  __shared__ int svar[kThreads];
+typedef double double2_u __attribute__((ext_vector_type(2), aligned(8)));
+__global__ __launch_bounds__(kThreads, 2) void k_bwd_rows(const SolveNode *sn,
+                                                             const int *slots,
+                                                             const int *wg_off, int nlvl,
+                                                             const double *x, int ldx, int nrhs,
+                                                             double *ws) {
+  constexpr int kSteps = 16;  // rows of a lane
+  __shared__ double red[kGroups][kRhsGroup][kBwdCols + 2];
   const int li = find_node_s(wg_off, nlvl, blockIdx.x);
   if (li < 0) return;
   const SolveNode &P = sn[slots[li]];
-  gcdouble *PL = (gcdouble *)P.L;
   gcint *Pperm = (gcint *)P.perm;
   gcint *Prows = (gcint *)P.rows;
   gdouble *part = (gdouble *)solve_P(ws, P, nrhs);  // count x nrhs x ne
@@ -565,56 +562,64 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rows_mr(const SolveNode *sn, c
   if (jend <= jbeg || r1 <= r0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ri = lane & 15, kq = lane >> 4;
-  {
-    const int i = r0 + tid;
-    svar[tid] = (i < r1) ? ((i < n) ? Pperm[i] : Prows[i - nd]) : 0;
-  }
-  __syncthreads();
-  const int nrow = r1 - r0;
-  // A operand: column acol of L (the lane's column of the wave's 16, clamped)
-  const int acol = imin(jbeg + 16 * wave + ri, jend - 1);
-  gcdouble *La = PL + (size_t)acol * ldl + r0;
-  for (int rc = 0; rc < nrhs; rc += 16 * NCH) {
-    const int nr = imin(16 * NCH, nrhs - rc);
-    mr_acc_t acc[NCH][kMrSplit];
+  const int i0 = r0 + 64 * wave;      // the wave's rows
+  const bool whole = i0 + 64 <= r1;
+  // A operand: this lane's column of each 16 (clamped), rows from 16 kq
+  gcdouble *La[4];
 #pragma unroll
-    for (int h = 0; h < NCH; ++h)
+  for (int t = 0; t < 4; ++t)
+    La[t] = (gcdouble *)P.L + (size_t)imin(jbeg + 16 * t + ri, jend - 1) * ldl + i0 + 16 * kq;
+  double av[4][kSteps];
+  if (whole) {
 #pragma unroll
-      for (int t = 0; t < kMrSplit; ++t) acc[h][t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < nrow; k0 += 4 * kSteps) {
-      double av[kSteps];
-      int vv[kSteps];
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int u = 0; u < kSteps; u += 2) {
+        const double2_u v = *(const double2_u __attribute__((address_space(1))) *)(La[t] + u);
+        av[t][u] = v.x;
+        av[t][u + 1] = v.y;
+      }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int u = 0; u < kSteps; ++u) {
-        const int kk = k0 + 4 * u + kq;
-        av[u] = masked(La[imin(kk, nrow - 1)], kk < nrow);
-        vv[u] = svar[imin(kk, nrow - 1)];
+        const int i = i0 + 16 * kq + u;
+        av[t][u] = masked(La[t][imin(i, r1 - 1) - i0 - 16 * kq], i < r1);
       }
+  }
+  int var[kSteps];  // variables of this lane's 16 rows (clamped)
 #pragma unroll
-      for (int h = 0; h < NCH; ++h) {
-        if (16 * h >= nr) break;
-        const int q = 16 * h + ri;
-        const double *xq = x + (size_t)(rc + imin(q, nr - 1)) * ldx;
-        double bv[kSteps];
+  for (int u = 0; u < kSteps; ++u) {
+    const int i = imin(i0 + 16 * kq + u, r1 - 1);
+    var[u] = (i < n) ? Pperm[i] : Prows[i - nd];
+  }
+  for (int rc = kRhsGroup * blockIdx.y; rc < nrhs; rc += kRhsGroup * gridDim.y) {
+    const int nr = imin(kRhsGroup, nrhs - rc);
+    const double *xq = x + (size_t)(rc + imin(ri, nr - 1)) * ldx;
+    double bv[kSteps];
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u)
-          bv[u] = masked(xq[vv[u]], q < nr && k0 + 4 * u + kq < nrow);
+    for (int u = 0; u < kSteps; ++u)
+      bv[u] = masked(xq[var[u]], ri < nr && i0 + 16 * kq + u < r1);
+    mr_acc_t acc[4];
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u)
-          acc[h][u % kMrSplit] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-              av[u], bv[u], acc[h][u % kMrSplit], 0, 0, 0);
-      }
-    }
-    // element (column kq + 4 rg of the wave's 16, right-hand side ri) of chunk h
+    for (int t = 0; t < 4; ++t) acc[t] = (mr_acc_t){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int h = 0; h < NCH; ++h)
+    for (int u = 0; u < kSteps; ++u)
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int c = 16 * wave + kq + 4 * rg, q = 16 * h + ri;
-        if (jbeg + c < jend && q < nr)
-          part[((size_t)local * nrhs + rc + q) * ne + jbeg + c] =
-              ((acc[h][0][rg] + acc[h][1][rg]) + acc[h][2][rg]) + acc[h][3][rg];
-      }
+      for (int t = 0; t < 4; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t][u], bv[u], acc[t], 0, 0, 0);
+    // element (column 16 t + kq + 4 rg of the chunk, right-hand side ri)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) red[wave][ri][16 * t + kq + 4 * rg] = acc[t][rg];
+    __syncthreads();
+    for (int q = wave; q < nr; q += kGroups)
+      if (jbeg + lane < jend)
+        part[((size_t)local * nrhs + rc + q) * ne + jbeg + lane] =
+            ((red[0][q][lane] + red[1][q][lane]) + red[2][q][lane]) + red[3][q][lane];
+    __syncthreads();
   }
 }
 
@@ -1187,14 +1192,9 @@ void launch_bwd(hipStream_t st, int nlvl, const SolveNode *sn, const int *slots,
                 int ldx, int nrhs, const int *rows_off, const int *chunk_off, int nwg,
                 double *ws, int dfuse, int ntri) {
   if (nlvl <= 0) return;
-  if (nwg > 0) {
-    if (nrhs <= 16)
-      hipLaunchKernelGGL(k_bwd_rows_mr<1>, dim3(nwg), dim3(kThreads), 0, st, sn, slots,
-                         chunk_off, nlvl, x, ldx, nrhs, ws);
-    else
-      hipLaunchKernelGGL(k_bwd_rows_mr<kMrChunks>, dim3(nwg), dim3(kThreads), 0, st, sn, slots,
-                         chunk_off, nlvl, x, ldx, nrhs, ws);
-  }
+  if (nwg > 0)
+    hipLaunchKernelGGL(k_bwd_rows, dim3(nwg, rhs_groups(nrhs, kRhsGroup)), dim3(kThreads), 0,
+                       st, sn, slots, chunk_off, nlvl, x, ldx, nrhs, ws);
   if (ntri <= 0) return;  // big fronts only
   if (nrhs == 1)
     hipLaunchKernelGGL(k_bwd_tri<1>, dim3(nlvl), dim3(kThreads), 0, st, sn, slots, rows_off, x,
