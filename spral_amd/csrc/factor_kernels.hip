@@ -1654,16 +1654,33 @@ __global__ __launch_bounds__(kThreads) void k_swap(NodeDev *nodes, const int *lv
 // so that many small fronts share each CU.
 constexpr int kTailWide = 1024, kTailNarrow = 256, kTailWideMaxFronts = 256;
 
+// The pivot search and elimination of one column at a time is a chain of
+// dependent passes over the trailing panel, so what bounds it is the number
+// of memory latencies and barriers a pivot takes.  Each pass issues its loads
+// together (clamped indices, a batch of eight a lane), the pivot columns stay in
+// LDS for the update, and the update's tiles (8 columns x 128 rows) are dealt
+// over the waves in both directions.  With one load at a time, the front's
+// pointers read again at each access and the update a column group at a time
+// over the whole workgroup, a pivot of a 300-column remainder took 26 us
+// (now under 7).
 template <int NT>
 struct TppShared {
-  double red[NT / 64];
-  int ired[NT / 64];
-  int flag;
+  static constexpr int kCap = (NT >= 1024) ? 2048 : 512;  // rows below a pivot kept in LDS
   // one candidate per wave (batched scan): result code, partner, 2x2 D^-1
   int code[NT / 64];
   int tt[NT / 64];
   double dd[3][NT / 64];
+  double red[NT / 64];
+  // the batch's rows: per row 64 partial results (largest, second largest,
+  // column of the largest with kBig set for an entry not below small)
+  double m1[NT / 64][64], m2[NT / 64][64];
+  int at[NT / 64][64];
+  double x[2][kCap], l[2][kCap];  // the pivot columns, and times D^-1
+  // rows [t0, n) of the columns APP eliminated: the row that position holds
+  static constexpr int kDefer = 1024;
+  int src[kDefer];
 };
+constexpr int kBig = 1 << 30;
 
 template <int NT>
 __device__ double wg_max(double v, TppShared<NT> &sh) {
@@ -1677,137 +1694,207 @@ __device__ double wg_max(double v, TppShared<NT> &sh) {
   return r;
 }
 
-template <int NT>
-__device__ int wg_and(int v, TppShared<NT> &sh) {
-  for (int off = 32; off > 0; off >>= 1) v &= __shfl_xor(v, off);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh.ired[threadIdx.x >> 6] = v;
-  __syncthreads();
-  int r = sh.ired[0];
-  for (int i = 1; i < NT / 64; ++i) r &= sh.ired[i];
-  __syncthreads();
-  return r;
-}
+// The fully-summed panel of a front
+struct Panel {
+  gdouble *L;
+  int ldl;
+  __device__ gdouble &operator()(int r, int c) const { return L[(size_t)c * ldl + r]; }
+};
 
-__device__ inline double &Lat(NodeDev &N, int r, int c) {
-  return N.L[(size_t)c * N.ldl + r];
-}
-
-// all |entries| of row/col idx within [from, to) below small?
-template <int NT>
-__device__ int tpp_col_small(NodeDev &N, int idx, int from, int to, double small,
-                             TppShared<NT> &sh) {
-  int ok = 1;
-  for (int c = from + threadIdx.x; c < idx; c += NT)
-    if (!(fabs(Lat(N, idx, c)) < small)) ok = 0;
-  for (int r = idx + threadIdx.x; r < to; r += NT)
-    if (!(fabs(Lat(N, r, idx)) < small)) ok = 0;
-  return wg_and(ok, sh);
-}
+constexpr int kTppLoads = 8;  // independent loads a lane issues in a scan
 
 template <int NT>
-__device__ double tpp_rc_max(NodeDev &N, int col, int nelim, int m, int skip,
-                             TppShared<NT> &sh) {
+__device__ double tpp_rc_max(const Panel &A, int col, int nelim, int m, TppShared<NT> &sh) {
   double best = 0.0;
-  for (int c = nelim + threadIdx.x; c < col; c += NT)
-    if (c != skip) best = fmax(best, fabs(Lat(N, col, c)));
-  for (int r = col + 1 + threadIdx.x; r < m; r += NT)
-    if (r != skip) best = fmax(best, fabs(Lat(N, r, col)));
+  for (int c = nelim + threadIdx.x; c < col; c += NT) best = fmax(best, fabs(A(col, c)));
+  for (int r = col + 1 + threadIdx.x; r < m; r += NT) best = fmax(best, fabs(A(r, col)));
   return wg_max(best, sh);
 }
 
+// Symmetric swap of rows/columns c1 and c2: the rows left of c1 from column cb
+// on, between c1 and c2 (a column against a row), and the columns below c2, as
+// one range.  src (or null): the deferred swaps of the columns before cb
 template <int NT>
-__device__ void tpp_swap(NodeDev &N, int c1, int c2, int m) {
+__device__ void tpp_swap(const Panel &A, int *perm, int cb, int *src, int c1, int c2, int m) {
   if (c1 == c2) return;
   if (c2 < c1) { int t = c1; c1 = c2; c2 = t; }
-  const int tid = threadIdx.x;
-  for (int c = tid; c < c1; c += NT) {
-    double t = Lat(N, c1, c); Lat(N, c1, c) = Lat(N, c2, c); Lat(N, c2, c) = t;
-  }
-  for (int i = c1 + 1 + tid; i < c2; i += NT) {
-    double t = Lat(N, i, c1); Lat(N, i, c1) = Lat(N, c2, i); Lat(N, c2, i) = t;
-  }
-  for (int r = c2 + 1 + tid; r < m; r += NT) {
-    double t = Lat(N, r, c1); Lat(N, r, c1) = Lat(N, r, c2); Lat(N, r, c2) = t;
+  const int tid = threadIdx.x, total = m - 2;
+  constexpr int kU = 2;
+  for (int i0 = cb + tid; i0 < total; i0 += kU * NT) {
+    gdouble *p[kU], *q[kU];
+    double vp[kU], vq[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = imin(i0 + u * NT, total - 1);
+      if (i < c1) {
+        p[u] = &A(c1, i);
+        q[u] = &A(c2, i);
+      } else if (i < c2 - 1) {
+        p[u] = &A(i + 1, c1);
+        q[u] = &A(c2, i + 1);
+      } else {
+        p[u] = &A(i + 2, c1);
+        q[u] = &A(i + 2, c2);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      vp[u] = *p[u];
+      vq[u] = *q[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (i0 + u * NT < total) {
+        *p[u] = vq[u];
+        *q[u] = vp[u];
+      }
   }
   if (tid == 0) {
-    double t = Lat(N, c1, c1); Lat(N, c1, c1) = Lat(N, c2, c2); Lat(N, c2, c2) = t;
-    int pt = N.perm[c1]; N.perm[c1] = N.perm[c2]; N.perm[c2] = pt;
-  }
-  __syncthreads();
-}
-
-constexpr int kTppCols = 8;  // trailing columns per pass of the TPP update
-
-template <int NT>
-__device__ void tpp_elim1(NodeDev &N, int k, int m, int n, double *ld) {
-  const double d11 = N.D[2 * k];
-  for (int r = k + 1 + threadIdx.x; r < m; r += NT) {
-    ld[r] = Lat(N, r, k);
-    Lat(N, r, k) = ld[r] * d11;
-  }
-  __syncthreads();
-  // trailing update, kTppCols columns per pass: a thread keeps its row's
-  // pivot entry in a register and issues the column loads together
-  for (int c0 = k + 1; c0 < n; c0 += kTppCols) {
-    double sc[kTppCols];
-#pragma unroll
-    for (int j = 0; j < kTppCols; ++j) sc[j] = (c0 + j < n) ? ld[c0 + j] : 0.0;
-    for (int r = c0 + threadIdx.x; r < m; r += NT) {
-      const double lk = Lat(N, r, k);
-      double v[kTppCols];
-#pragma unroll
-      for (int j = 0; j < kTppCols; ++j)
-        v[j] = (c0 + j < n && r >= c0 + j) ? Lat(N, r, c0 + j) : 0.0;
-#pragma unroll
-      for (int j = 0; j < kTppCols; ++j)
-        if (c0 + j < n && r >= c0 + j) Lat(N, r, c0 + j) = v[j] - lk * sc[j];
+    const double t = A(c1, c1);
+    A(c1, c1) = A(c2, c2);
+    A(c2, c2) = t;
+    const int pt = perm[c1];
+    perm[c1] = perm[c2];
+    perm[c2] = pt;
+    if (src) {
+      const int st = src[c1 - cb];
+      src[c1 - cb] = src[c2 - cb];
+      src[c2 - cb] = st;
     }
   }
-  if (threadIdx.x == 0) Lat(N, k, k) = 1.0;
   __syncthreads();
 }
 
-template <int NT>
-__device__ void tpp_elim2(NodeDev &N, int k, int m, int n, double *ld, double *ld2) {
-  const double d11 = N.D[2 * k], d21 = N.D[2 * k + 1], d22 = N.D[2 * k + 3];
-  for (int r = k + 2 + threadIdx.x; r < m; r += NT) {
-    double x1 = Lat(N, r, k), x2 = Lat(N, r, k + 1);
-    ld[r] = x1;
-    ld2[r] = x2;
-    Lat(N, r, k) = d11 * x1 + d21 * x2;
-    Lat(N, r, k + 1) = d21 * x1 + d22 * x2;
+// The deferred row swaps of the columns before t0: rows [t0, t0 + cnt) of each
+// column in the order of src, U 64-row pieces; a wave takes NC columns at a time
+// (16 loads on their way)
+template <int NT, int NC>
+__device__ void tpp_rows(const Panel &A, const int *src, int t0, int cnt) {
+  constexpr int U = TppShared<NT>::kDefer / 64 / NC;
+  const int lane = threadIdx.x & 63;
+  int from[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) from[u] = t0 + src[imin(64 * u + lane, cnt - 1)];
+  for (int c = NC * uni((int)threadIdx.x >> 6); c < t0; c += NC * (NT / 64)) {
+    double v[NC][U];
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[k][u] = A(from[u], imin(c + k, t0 - 1));
+    __builtin_amdgcn_s_waitcnt(0);  // the columns are read before they are written
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+      if (c + k < t0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (64 * u + lane < cnt) A(t0 + 64 * u + lane, c + k) = v[k][u];
+      }
+  }
+}
+
+constexpr int kTppCols = 8, kTppRows = 128;  // a wave's tile of the TPP update
+
+// Elimination by pivot k (W = 1: D^{-1} = d0; W = 2: [d0 d1; d1 d3] on k, k+1):
+// the rows below scaled, then columns [k + W, n) minus their products.  x and l
+// hold the unscaled and the scaled pivot columns of row r at r - k - W; in LDS,
+// or for longer columns x in the front's workspace and l in the panel.
+template <int NT, int W, bool LDS>
+__device__ void tpp_elim(const Panel &A, int k, int m, int n, double d0, double d1, double d3,
+                         TppShared<NT> &sh, gdouble *w0, gdouble *w1) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int base = k + W;
+  for (int r = base + tid; r < m; r += NT) {
+    const int i = r - base;
+    const double x0 = A(r, k);
+    if (W == 1) {
+      const double l0 = x0 * d0;
+      A(r, k) = l0;
+      if (LDS) {
+        sh.x[0][i] = x0;
+        sh.l[0][i] = l0;
+      } else {
+        w0[i] = x0;
+      }
+    } else {
+      const double x1 = A(r, k + 1);
+      const double l0 = d0 * x0 + d1 * x1, l1 = d1 * x0 + d3 * x1;
+      A(r, k) = l0;
+      A(r, k + 1) = l1;
+      if (LDS) {
+        sh.x[0][i] = x0;
+        sh.x[1][i] = x1;
+        sh.l[0][i] = l0;
+        sh.l[1][i] = l1;
+      } else {
+        w0[i] = x0;
+        w1[i] = x1;
+      }
+    }
   }
   __syncthreads();
-  for (int c0 = k + 2; c0 < n; c0 += kTppCols) {
-    double s1[kTppCols], s2[kTppCols];
+  const int G = idiv_up(n - base, kTppCols), RB = idiv_up(m - base, kTppRows);
+  for (int t = wave; t < G * RB; t += NT / 64) {
+    const int rb = t / G, c0 = base + (t - rb * G) * kTppCols;
+    const int r0 = c0 + rb * kTppRows;
+    if (r0 >= m) continue;
+    double s0[kTppCols], s1[kTppCols];
 #pragma unroll
     for (int j = 0; j < kTppCols; ++j) {
-      s1[j] = (c0 + j < n) ? ld[c0 + j] : 0.0;
-      s2[j] = (c0 + j < n) ? ld2[c0 + j] : 0.0;
+      const int i = imin(c0 + j, n - 1) - base;
+      s0[j] = LDS ? sh.x[0][i] : w0[i];
+      if (W == 2) s1[j] = LDS ? sh.x[1][i] : w1[i];
     }
-    for (int r = c0 + threadIdx.x; r < m; r += NT) {
-      const double l1 = Lat(N, r, k), l2 = Lat(N, r, k + 1);
-      double v[kTppCols];
 #pragma unroll
-      for (int j = 0; j < kTppCols; ++j)
-        v[j] = (c0 + j < n && r >= c0 + j) ? Lat(N, r, c0 + j) : 0.0;
+    for (int h = 0; h < kTppRows / 64; h += 2) {
+      double v[2][kTppCols], l0[2], l1[2];
 #pragma unroll
-      for (int j = 0; j < kTppCols; ++j)
-        if (c0 + j < n && r >= c0 + j) Lat(N, r, c0 + j) = v[j] - (l1 * s1[j] + l2 * s2[j]);
+      for (int g = 0; g < 2; ++g) {
+        const int r = imin(r0 + 64 * (h + g) + lane, m - 1);
+        l0[g] = LDS ? sh.l[0][r - base] : A(r, k);
+        if (W == 2) l1[g] = LDS ? sh.l[1][r - base] : A(r, k + 1);
+#pragma unroll
+        for (int j = 0; j < kTppCols; ++j) v[g][j] = A(r, imin(c0 + j, n - 1));
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int r = r0 + 64 * (h + g) + lane;
+#pragma unroll
+        for (int j = 0; j < kTppCols; ++j)
+          if (c0 + j < n && r >= c0 + j && r < m)
+            A(r, c0 + j) = v[g][j] - (W == 1 ? l0[g] * s0[j] : l0[g] * s0[j] + l1[g] * s1[j]);
+      }
     }
   }
-  if (threadIdx.x == 0) {
-    Lat(N, k, k) = 1.0;
-    Lat(N, k + 1, k) = 0.0;
-    Lat(N, k + 1, k + 1) = 1.0;
+  if (tid == 0) {
+    A(k, k) = 1.0;
+    if (W == 2) {
+      A(k + 1, k) = 0.0;
+      A(k + 1, k + 1) = 1.0;
+    }
   }
   __syncthreads();
 }
 
-// One TPP candidate p (> nelim) tested by one wave, reading the panel only
-// (the tests of a scan are read-only, so the waves of a workgroup test
-// consecutive candidates at once and the first that passes is taken, as a
+// Whether every entry of column k at and below the diagonal is below small
+// (one wave; NaN is not)
+__device__ inline bool tpp_wave_small(const Panel &A, int k, int m, double small) {
+  const int lane = threadIdx.x & 63;
+  int big = 0;
+  for (int r0 = k; r0 < m; r0 += 64 * kTppLoads) {
+    double v[kTppLoads];
+#pragma unroll
+    for (int u = 0; u < kTppLoads; ++u) v[u] = A(imin(r0 + 64 * u + lane, m - 1), k);
+#pragma unroll
+    for (int u = 0; u < kTppLoads; ++u)
+      if (!(fabs(v[u]) < small)) big = 1;
+  }
+  return __ballot(big) == 0;
+}
+
+// A batch of TPP candidates p0, p0 + 1, ..., one per wave, tested reading the
+// panel only (the tests of a scan are read-only, so the waves of a workgroup
+// test consecutive candidates at once and the first that passes is taken, as a
 // one-at-a-time scan would).  The decisions are those of the scan's steps
 // (ldlt_tpp.cxx:192-259): a zero row/column; else t = the first largest
 // |a(p, c)|, c in [nelim, p), the 2x2 test on (t, p) against the largest
@@ -1815,33 +1902,79 @@ __device__ void tpp_elim2(NodeDev &N, int k, int m, int n, double *ld, double *l
 // row p and column p give the zero test, t, row p's largest entry other
 // than t (its second largest: t holds the first largest) and column p's
 // largest; row t and column t give t's largest other than p.  Every maximum
-// is exact, so the decision equals the one-at-a-time scan's.  Returns the
-// code (0 fail, 1 zero column, 2 2x2, 3 1x1), wave-uniform; t and the 2x2
-// D^-1 in the out arguments.
-__device__ inline int tpp_wave_test(NodeDev &N, int p, int nelim, int m, double u,
+// is exact, so the decision equals the one-at-a-time scan's.
+//
+// The batch's rows are consecutive, so the whole workgroup reads them column
+// by column, a 128-byte piece (16 rows) at a time: a wave reading its own row
+// touches a line per entry, 64 a load.
+template <int NT>
+__device__ inline void tpp_batch_rows(const Panel &A, int p0, int nelim, int n, double small,
+                                      TppShared<NT> &sh) {
+  constexpr int NW = NT / 64, kU = kTppLoads;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane & (NW - 1), part = wave * (64 / NW) + lane / NW;  // of 64 columns
+  const int p = imin(p0 + row, n - 1);
+  double m1 = -1.0, m2 = -1.0;
+  int at = kBig - 1, big = 0;
+  for (int o = nelim + part; o < p0 + NW; o += 64 * kU) {
+    double v[kU];
+#pragma unroll
+    for (int k = 0; k < kU; ++k) v[k] = A(p, imin(o + 64 * k, p - 1));
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      const int c = o + 64 * k;
+      const double w = fabs(v[k]);
+      if (c < p) {
+        if (!(w < small)) big = kBig;
+        if (w > m1) {
+          m2 = m1;
+          m1 = w;
+          at = c;
+        } else if (w > m2) {
+          m2 = w;
+        }
+      }
+    }
+  }
+  sh.m1[row][part] = m1;
+  sh.m2[row][part] = m2;
+  sh.at[row][part] = at | big;
+}
+
+// The test of candidate p, row of the batch's rows, by one wave, vc the first
+// loads of its column.  Returns the code (0 fail, 1 zero column, 2 2x2, 3 1x1),
+// wave-uniform; t and the 2x2 D^-1 in the out arguments.
+template <int NT>
+__device__ inline int tpp_wave_test(const Panel &A, int p, int row, const TppShared<NT> &sh,
+                                    const double (&vc)[kTppLoads], int nelim, int m, double u,
                                     double small, int &t_out, double &d0, double &d1,
                                     double &d3) {
   const int lane = threadIdx.x & 63;
+  constexpr int kU = kTppLoads;
+  const double a22 = uni(vc[0]);  // (lane 0's)
   // pass A: row p over [nelim, p) and column p over [p, m)
-  int big = 0;                        // some |entry| not below small (NaN counts)
-  double m1 = -1.0, m2 = -1.0;        // row p: largest, second largest (-1: none)
-  int a1 = INT_MAX;                   // first column holding m1
-  for (int c = nelim + lane; c < p; c += 64) {
-    const double v = fabs(Lat(N, p, c));
-    if (!(v < small)) big = 1;
-    if (v > m1) {
-      m2 = m1;
-      m1 = v;
-      a1 = c;
-    } else if (v > m2) {
-      m2 = v;
-    }
-  }
+  double m1 = sh.m1[row][lane], m2 = sh.m2[row][lane];  // largest, second (-1: none)
+  int a1 = sh.at[row][lane];          // first column holding m1
+  int big = a1 & kBig;                // some |entry| not below small (NaN counts)
+  a1 &= ~kBig;
   double cp = 0.0;                    // column p below the diagonal
-  for (int r = p + lane; r < m; r += 64) {
-    const double v = fabs(Lat(N, r, p));
-    if (!(v < small)) big = 1;
-    if (r > p) cp = fmax(cp, v);
+  auto column = [&](const double (&v)[kU], int o) {
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      const int r = p + o + 64 * k + lane;
+      const double w = fabs(v[k]);
+      if (r < m) {
+        if (!(w < small)) big = 1;
+        if (r > p) cp = fmax(cp, w);
+      }
+    }
+  };
+  column(vc, 0);
+  for (int o = 64 * kU; o < m - p; o += 64 * kU) {
+    double v[kU];
+#pragma unroll
+    for (int k = 0; k < kU; ++k) v[k] = A(imin(p + o + 64 * k + lane, m - 1), p);
+    column(v, o);
   }
   for (int off = 32; off > 0; off >>= 1) {
     const double om1 = __shfl_xor(m1, off), om2 = __shfl_xor(m2, off);
@@ -1857,31 +1990,44 @@ __device__ inline int tpp_wave_test(NodeDev &N, int p, int nelim, int m, double 
   }
   if (!__ballot(big)) return 1;
   // t: the first largest of row p (nelim when every entry is NaN)
-  const int t = (a1 == INT_MAX) ? nelim : __builtin_amdgcn_readfirstlane(a1);
+  const int t = (a1 == kBig - 1) ? nelim : __builtin_amdgcn_readfirstlane(a1);
   t_out = t;
   // maxp = rc_max(p, skip t): row p without column t, column p below
-  double maxp = fmax(fmax(0.0, (a1 == INT_MAX) ? -1.0 : m2), cp);
-  // pass B: maxt = rc_max(t, skip p): row t over [nelim, t), column t over
-  // (t, m) without row p
-  double mt = 0.0;
-  for (int c = nelim + lane; c < t; c += 64) mt = fmax(mt, fabs(Lat(N, t, c)));
-  for (int r = t + 1 + lane; r < m; r += 64)
-    if (r != p) mt = fmax(mt, fabs(Lat(N, r, t)));
-  for (int off = 32; off > 0; off >>= 1) mt = fmax(mt, __shfl_xor(mt, off));
-  const double maxt = uni(mt);
+  double maxp = fmax(fmax(0.0, (a1 == kBig - 1) ? -1.0 : m2), cp);
   maxp = uni(maxp);
+  const double a11 = A(t, t), a21 = A(p, t);
   // 2x2 test (t < p)
-  const double a11 = Lat(N, t, t), a21 = Lat(N, p, t), a22 = Lat(N, p, p);
   const double maxpiv = fmax(fabs(a11), fmax(fabs(a21), fabs(a22)));
   if (!(maxpiv < small)) {
     const double detscale = 1 / maxpiv;
     const double det0 = (a11 * detscale) * a22;
     const double det1 = (a21 * detscale) * a21;
     const double det = det0 - det1;
-    if (!(fabs(det) < fmax(small, fmax(fabs(det0 / 2), fabs(det1 / 2))))) {
-      const double e0 = (a22 * detscale) / det;
-      const double e1 = (-a21 * detscale) / det;
-      const double e3 = (a11 * detscale) / det;
+    const double e0 = (a22 * detscale) / det;
+    const double e1 = (-a21 * detscale) / det;
+    const double e3 = (a11 * detscale) / det;
+    // (pass B only where its result can matter: maxt only adds to the sums)
+    if (!(fabs(det) < fmax(small, fmax(fabs(det0 / 2), fabs(det1 / 2)))) &&
+        (maxp < small || u * fmax(fabs(e1) * maxp, fabs(e3) * maxp) < 1.0)) {
+      // pass B: maxt = rc_max(t, skip p): row t over [nelim, t), column t over
+      // (t, m) without row p
+      double mt = 0.0;
+      for (int o = 0; o < imax(t - nelim, m - t - 1); o += 64 * kU) {
+        double vr[kU], vt[kU];
+#pragma unroll
+        for (int k = 0; k < kU; ++k)
+          vr[k] = A(t, imax(imin(nelim + o + 64 * k + lane, t - 1), 0));
+#pragma unroll
+        for (int k = 0; k < kU; ++k) vt[k] = A(imin(t + 1 + o + 64 * k + lane, m - 1), t);
+#pragma unroll
+        for (int k = 0; k < kU; ++k) {
+          const int c = nelim + o + 64 * k + lane, r = t + 1 + o + 64 * k + lane;
+          if (c < t) mt = fmax(mt, fabs(vr[k]));
+          if (r < m && r != p) mt = fmax(mt, fabs(vt[k]));
+        }
+      }
+      for (int off = 32; off > 0; off >>= 1) mt = fmax(mt, __shfl_xor(mt, off));
+      const double maxt = uni(mt);
       bool ok2;
       if (fmax(maxp, maxt) < small) {
         ok2 = true;
@@ -1905,8 +2051,7 @@ __device__ inline int tpp_wave_test(NodeDev &N, int p, int nelim, int m, double 
 // TPP on the columns [nelim, n) that APP left, by the whole workgroup;
 // returns the new nelim (uniform) and stores it in N.nelim.
 template <int NT>
-__device__ int tpp_front(NodeDev &N, const FactorParams &fp, int nelim, TppShared<NT> &sh,
-                         int &s_t) {
+__device__ int tpp_front(NodeDev &N, const FactorParams &fp, int nelim, TppShared<NT> &sh) {
   const int n = N.n, m = N.m;
   if (nelim >= n) return nelim;
   // as factor_node_indef (src/ssids/cpu/factor.hxx:77-80): TPP finishes a
@@ -1914,28 +2059,71 @@ __device__ int tpp_front(NodeDev &N, const FactorParams &fp, int nelim, TppShare
   // method or the failed-pivot method is TPP
   if (!(fp.pivot_tpp || m == n || fp.tpp_failed)) return nelim;
   const double u = fp.u, small = fp.small;
-  double *ld = N.bak, *ld2 = N.bak + N.ldbak;
-  const int tid = threadIdx.x;
-  while (nelim < n) {
-    if (tpp_col_small(N, nelim, nelim, m, small, sh)) {
-      if (!fp.action) { if (tid == 0) N.flag = -5; return nelim; }
-      for (int r = nelim + tid; r < m; r += NT) Lat(N, r, nelim) = 0.0;
-      if (tid == 0) { N.D[2 * nelim] = 0.0; N.D[2 * nelim + 1] = 0.0; N.nzero++; }
-      __syncthreads();
-      ++nelim;
-      continue;
+  const Panel A{(gdouble *)N.L, N.ldl};
+  gdouble *D = (gdouble *)N.D, *w0 = (gdouble *)N.bak, *w1 = w0 + N.ldbak;
+  int *perm = N.perm;
+  const int tid = threadIdx.x, lane = tid & 63, wv = uni(tid >> 6);
+  // the row swaps of the columns before t0 wait until the end: they are most of
+  // a swap where few of many columns are left (1,500 of 1,800 at a KKT root)
+  const int t0 = nelim, cnt = n - t0;
+  const bool defer = cnt <= TppShared<NT>::kDefer;
+  const int cb = defer ? t0 : 0;
+  int *src = defer ? sh.src : nullptr;
+  if (defer)
+    for (int i = tid; i < cnt; i += NT) sh.src[i] = i;
+  bool swapped = false, failed = false;
+  auto swap = [&](int c1, int c2) {
+    swapped = swapped || c1 != c2;
+    tpp_swap<NT>(A, perm, cb, src, c1, c2, m);
+  };
+  __syncthreads();
+  auto zero_pivot = [&] {
+    for (int r = nelim + tid; r < m; r += NT) A(r, nelim) = 0.0;
+    if (tid == 0) {
+      D[2 * nelim] = 0.0;
+      D[2 * nelim + 1] = 0.0;
+      N.nzero++;
     }
-    int done = 0;
+    __syncthreads();
+    ++nelim;
+  };
+  auto pivot1 = [&] {
+    const double d = 1.0 / A(nelim, nelim);
+    if (tid == 0) {
+      D[2 * nelim] = d;
+      D[2 * nelim + 1] = 0.0;
+    }
+    if (m - nelim - 1 <= TppShared<NT>::kCap)
+      tpp_elim<NT, 1, true>(A, nelim, m, n, d, 0.0, 0.0, sh, w0, w1);
+    else
+      tpp_elim<NT, 1, false>(A, nelim, m, n, d, 0.0, 0.0, sh, w0, w1);
+    nelim += 1;
+  };
+  while (nelim < n) {
     // candidates nelim+1, nelim+2, ... in batches of one per wave; the first
-    // that passes in order is taken
+    // that passes in order is taken.  In the first batch the last wave tests
+    // column nelim for a zero pivot, which goes before any candidate.
     constexpr int NW = NT / 64;
-    const int wv = threadIdx.x >> 6;
-    for (int base = nelim + 1; base < n && !done; base += NW) {
-      const int pc = base + wv;
+    int c = 0, t = 0, p = 0;
+    double d0 = 0.0, d1 = 0.0, d3 = 0.0;
+    for (int base = nelim + 1, nc = NW - 1;;) {
+      const bool first = nc < NW;
       int code = 0, tw = 0;
       double e0 = 0.0, e1 = 0.0, e3 = 0.0;
-      if (pc < n) code = tpp_wave_test(N, pc, nelim, m, u, small, tw, e0, e1, e3);
-      if ((tid & 63) == 0) {
+      const int pw = imin(base + wv, n - 1);
+      double vc[kTppLoads];
+      if (base < n) {
+        if (wv < nc) {
+#pragma unroll
+          for (int k = 0; k < kTppLoads; ++k) vc[k] = A(imin(pw + 64 * k + lane, m - 1), pw);
+        }
+        tpp_batch_rows<NT>(A, base, nelim, n, small, sh);
+      }
+      if (wv == nc) code = tpp_wave_small(A, nelim, m, small) ? 1 : 0;  // the first batch
+      __syncthreads();
+      if (wv < nc && base + wv < n)
+        code = tpp_wave_test<NT>(A, pw, wv, sh, vc, nelim, m, u, small, tw, e0, e1, e3);
+      if (lane == 0) {
         sh.code[wv] = code;
         sh.tt[wv] = tw;
         sh.dd[0][wv] = e0;
@@ -1943,72 +2131,66 @@ __device__ int tpp_front(NodeDev &N, const FactorParams &fp, int nelim, TppShare
         sh.dd[2][wv] = e3;
       }
       __syncthreads();
-      int w0 = -1;
-      for (int v = 0; v < NW; ++v)
-        if (sh.code[v] != 0) {
-          w0 = v;
-          break;
-        }
-      int c = 0, t = 0;
-      double d0 = 0.0, d1 = 0.0, d3 = 0.0;
-      if (w0 >= 0) {
-        c = sh.code[w0];
-        t = sh.tt[w0];
-        d0 = sh.dd[0][w0];
-        d1 = sh.dd[1][w0];
-        d3 = sh.dd[2][w0];
-      }
-      __syncthreads();  // every thread has read the batch before it is reused
-      if (w0 < 0) continue;
-      const int p = base + w0;
-      done = 1;
-      if (c == 1) {  // a zero row/column: a zero pivot at nelim
-        if (!fp.action) { if (tid == 0) N.flag = -5; return nelim; }
-        tpp_swap<NT>(N, p, nelim, m);
-        for (int r = nelim + tid; r < m; r += NT) Lat(N, r, nelim) = 0.0;
-        if (tid == 0) { N.D[2 * nelim] = 0.0; N.D[2 * nelim + 1] = 0.0; N.nzero++; }
-        __syncthreads();
-        ++nelim;
-      } else if (c == 2) {
-        tpp_swap<NT>(N, t, nelim, m);
-        tpp_swap<NT>(N, p, nelim + 1, m);
-        if (tid == 0) {
-          N.D[2 * nelim] = d0;
-          N.D[2 * nelim + 1] = d1;
-          N.D[2 * nelim + 2] = INFINITY;
-          N.D[2 * nelim + 3] = d3;
-        }
-        __syncthreads();
-        tpp_elim2<NT>(N, nelim, m, n, ld, ld2);
-        nelim += 2;
-      } else {
-        tpp_swap<NT>(N, p, nelim, m);
-        if (tid == 0) {
-          N.D[2 * nelim] = 1.0 / Lat(N, nelim, nelim);
-          N.D[2 * nelim + 1] = 0.0;
-        }
-        __syncthreads();
-        tpp_elim1<NT>(N, nelim, m, n, ld);
-        nelim += 1;
-      }
-    }
-    if (!done) {
-      const int p = nelim;
-      double maxp = tpp_rc_max(N, p, nelim, m, -1, sh);
-      if (fabs(Lat(N, p, p)) >= u * maxp) {
-        if (tid == 0) {
-          N.D[2 * nelim] = 1.0 / Lat(N, nelim, nelim);
-          N.D[2 * nelim + 1] = 0.0;
-        }
-        __syncthreads();
-        tpp_elim1<NT>(N, nelim, m, n, ld);
-        nelim += 1;
-      } else {
+      const unsigned long long hit = __ballot(lane < NW && sh.code[lane & (NW - 1)] != 0);
+      if (first && ((hit >> nc) & 1)) {
+        c = 1;
+        p = nelim;
         break;
       }
+      const unsigned long long cand = hit & ((1ull << nc) - 1);
+      if (cand != 0) {
+        const int w = __builtin_ctzll(cand);
+        p = base + w;
+        c = sh.code[w];
+        t = sh.tt[w];
+        d0 = sh.dd[0][w];
+        d1 = sh.dd[1][w];
+        d3 = sh.dd[2][w];
+        break;
+      }
+      base += nc;
+      nc = NW;
+      if (base >= n) break;
+      __syncthreads();  // every thread has read the batch before it is reused
+    }
+    __syncthreads();  // (as above)
+    if (c == 1) {  // a zero row/column: a zero pivot at nelim
+      if (!fp.action) {
+        if (tid == 0) N.flag = -5;
+        failed = true;
+        break;
+      }
+      swap(p, nelim);
+      zero_pivot();
+    } else if (c == 2) {
+      swap(t, nelim);
+      swap(p, nelim + 1);
+      if (tid == 0) {
+        D[2 * nelim] = d0;
+        D[2 * nelim + 1] = d1;
+        D[2 * nelim + 2] = INFINITY;
+        D[2 * nelim + 3] = d3;
+      }
+      if (m - nelim - 2 <= TppShared<NT>::kCap)
+        tpp_elim<NT, 2, true>(A, nelim, m, n, d0, d1, d3, sh, w0, w1);
+      else
+        tpp_elim<NT, 2, false>(A, nelim, m, n, d0, d1, d3, sh, w0, w1);
+      nelim += 2;
+    } else if (c == 3) {
+      swap(p, nelim);
+      pivot1();
+    } else {  // no candidate: 1x1 on column nelim itself, or the end
+      const double maxp = tpp_rc_max(A, nelim, nelim, m, sh);
+      if (!(fabs(A(nelim, nelim)) >= u * maxp)) break;
+      pivot1();
     }
   }
-  if (tid == 0) N.nelim = nelim;
+  if (defer && swapped) {
+    if (cnt <= 64 * 4) tpp_rows<NT, 4>(A, sh.src, t0, cnt);
+    else if (cnt <= 64 * 8) tpp_rows<NT, 2>(A, sh.src, t0, cnt);
+    else tpp_rows<NT, 1>(A, sh.src, t0, cnt);
+  }
+  if (tid == 0 && !failed) N.nelim = nelim;
   return nelim;
 }
 
@@ -2030,7 +2212,6 @@ template <int NT>
 __global__ __launch_bounds__(NT) void k_tail(NodeDev *nodes, const int *lvl_slots,
                                                    FactorParams fp, int *scratch) {
   __shared__ TppShared<NT> sh;
-  __shared__ int s_t;
   NodeDev &N = nodes[lvl_slots[blockIdx.x]];
   const int tid = threadIdx.x;
   int nelim;
@@ -2049,7 +2230,7 @@ __global__ __launch_bounds__(NT) void k_tail(NodeDev *nodes, const int *lvl_slot
     __syncthreads();
   }
   const int t0 = nelim;  // APP pivots end here
-  nelim = tpp_front(N, fp, nelim, sh, s_t);
+  nelim = tpp_front(N, fp, nelim, sh);
   __syncthreads();
   // Dd
   for (int k = tid; k < nelim; k += NT) {
