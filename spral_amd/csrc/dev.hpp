@@ -166,6 +166,30 @@ __device__ inline int table_find(const int *off, int n, int b) {
   return lo;
 }
 
+// The front of a level's workgroup b: index li of its table segment (as
+// table_find) and the number of workgroups before it.  A level of one front
+// needs no table: the caller checks its workgroup against the front's own work.
+__device__ inline int front_of(const int *off, int n, int b, int &before) {
+  before = 0;
+  if (n == 1) return 0;
+  const int li = table_find(off, n, b);
+  if (li >= 0) before = off[li];
+  return li;
+}
+
+// The uniform values are loaded by here, together.  A kernel's first loads each
+// take the better part of a microsecond (the caches are cold at its start), and
+// the compiler moves a load behind the early return that does not need it.
+template <class T>
+__device__ inline void loaded(const T &v) {
+  asm volatile("" ::"s"(v));
+}
+template <class T, class... U>
+__device__ inline void loaded(const T &v, const U &...rest) {
+  loaded(v);
+  loaded(rest...);
+}
+
 // v if keep, else +0.0.  The value passes through an empty asm first, so the
 // selection is not turned into a branch around the load that produced it
 // (which would serialize a batch of loads behind their uses).

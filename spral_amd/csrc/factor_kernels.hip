@@ -40,10 +40,6 @@ typedef unsigned uint16v_t __attribute__((ext_vector_type(16)));
 
 // front of workgroup b in a level table, or -1 past the table's total (grids
 // sized for the plan's capacities may be larger than the level needs)
-__device__ inline int find_node(const int *wg_off, int nlvl, int b) {
-  return table_find(wg_off, nlvl, b);
-}
-
 // element (i,j), i>=j, of the front (panel for j<n, contribution block else)
 __device__ inline double *front_at(const NodeDev &N, int i, int j) {
   if (j < N.n) return N.L + (size_t)j * N.ldl + i;
@@ -303,7 +299,7 @@ constexpr int kGT = 64;  // gather tile edge
 
 template <int PART, typename CT>
 __device__ __forceinline__ int gather_tile(
-    NodeDev *nodes, const int *lvl_slots, const int *wg_off, int nlvl,
+    NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
     const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int (&mr)[kGT],
     int (&mc)[kGT]);
@@ -327,7 +323,7 @@ struct GatherArgs {  // the level's gather inputs (a pivot launch that assembles
 // twice as many workgroups on a CU.
 // C32 (FIRST only): the children's contribution blocks are FP32
 template <int NW, bool FIRST, bool C32>
-__global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, int s0,
                                                   int step, FactorParams fp, GatherArgs ga) {
   constexpr int R = kBlk / NW;
   static_assert(NW == kDiagWaves && R == kDiagCols, "a row of lanes holds L of a wave's columns");
@@ -349,12 +345,12 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
     static_assert(kGT == kBlk, "the gather tile is the pivot block's staging array");
     // the tile's LDS is the pivot block's own (t, lp, inv_lp), used in turn
     typedef typename std::conditional<C32, float, double>::type CT;
-    s = gather_tile<1, CT>(nodes, lvl_slots, ga.wg_off, ga.nlvl, ga.child_list, ga.aval,
+    s = gather_tile<1, CT>(nodes, s0, ga.wg_off, ga.nlvl, ga.child_list, ga.aval,
                            ga.asrc, ga.arow, ga.acix, ga.scaling, t, lp, inv_lp);
     if (s < 0) return;
     __syncthreads();  // the block's stores are visible to the whole workgroup
   } else {
-    s = lvl_slots[blockIdx.x];
+    s = s0 + blockIdx.x;
   }
   NodeDev &N = nodes[s];
   if (step >= N.nsteps) return;
@@ -654,23 +650,24 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, const int *lvl
 // maxima kept as values, each workgroup reduced 64 columns by shuffles and
 // made 256 atomics on the front's 64 words.)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, int s0,
                                                     const int *wg_off, int nlvl, int step,
                                                     FactorParams fp) {
   // M = L_bb^{-1} (or the left-rows chunk)
   __shared__ double ms[kBlk][kBlk + 1];
   __shared__ double dv[2 * kBlk + 2];
   __shared__ int lps[kBlk];
-  const int li = find_node(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return;
-  NodeDev &N = nodes[lvl_slots[li]];
-  if (step >= N.nsteps) return;
-  const int p = N.p, w = N.w;
-  if (w == 0) return;
-  int local = blockIdx.x - wg_off[li];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ldl = N.ldl;
+  NodeDev &N = nodes[s0 + li];
+  const int nsteps = N.nsteps, p = N.p, w = N.w, ldl = N.ldl, m = N.m;
   double *L = N.L;
+  const double *NW = N.W, *ND = N.D;
+  loaded(nsteps, p, w, ldl, m, L, NW, ND);
+  int local = blockIdx.x - before;
+  if (step >= nsteps || w == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the first nleft workgroups permute rows p..p+w-1 of the eliminated
   // columns left of p into the block's elimination order (64-column chunks)
   const int nleft = step;  // upper bound on ceil(p / 64)
@@ -696,11 +693,11 @@ __global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int
   }
   local -= nleft;
   // ---- rows [rb, rb+64) below the block: X^T = M A21[:, lp]^T on MFMA
-  const int r0 = p + w, m = N.m;
+  const int r0 = p + w;
   const int rb = r0 + local * kBlk;
   if (rb >= m) return;
-  gcdouble *Wg = (gcdouble *)N.W;
-  gcdouble *Dg = (gcdouble *)N.D;
+  gcdouble *Wg = (gcdouble *)NW;
+  gcdouble *Dg = (gcdouble *)ND;
   gcint *lpg = (gcint *)N.lp;
   double wv[kBlk / 4];
 #pragma unroll
@@ -810,9 +807,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_apply(NodeDev *nodes, const int
 
 // number of block pivots that pass the threshold test (split 2x2 avoided):
 // the first column holding an |l| above 1/u; wave-uniform.
-__device__ inline int block_npass(const NodeDev &N) {
-  const int w = N.w, p = N.p;
-  const unsigned long long fail = __atomic_load_n(&N.fail, __ATOMIC_RELAXED);
+__device__ inline int block_npass(const NodeDev &N, int p, int w, unsigned long long fail) {
   int np = fail ? __ffsll((long long)fail) - 1 : w;
   if (np > 0 && np < w) {
     double d11 = N.D[2 * (p + np - 1)], d21 = N.D[2 * (p + np - 1) + 1];
@@ -869,17 +864,19 @@ __device__ inline void tile_of(int tile, int TI, int TJ, int &I, int &J) {
   I = J + (tile - first(J));
 }
 
-__global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, int s0,
                                                      const int *wg_off, int nlvl, int step,
                                                      int mode, FactorParams fp) {
   // 32-pivot K chunks: the two operand tiles take 34 KB, four workgroups a CU
   constexpr int kUpdK = 32;
   __shared__ double As[kTile][kUpdK + 1];
   __shared__ double Bs[kTile][kUpdK + 1];
-  const int li = find_node(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return;
-  NodeDev &N = nodes[lvl_slots[li]];
-  const int local = blockIdx.x - wg_off[li], count = wg_off[li + 1] - wg_off[li];
+  NodeDev &N = nodes[s0 + li];
+  const int local = blockIdx.x - before, count = wg_off[li + 1] - before;
+  if (local >= count) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int a0, K, t0, cend, fa, fb, p = 0, w = 0;
   if (mode == 0) {
@@ -887,7 +884,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_update(NodeDev *nodes, const in
     p = N.p;
     w = N.w;
     if (w == 0) return;
-    int np = fp.posdef ? N.w : block_npass(N);
+    int np = fp.posdef ? N.w : block_npass(N, p, w, N.fail);
     if (local == 0 && tid == 0) N.npass = np;
     a0 = p;
     K = np;
@@ -1124,30 +1121,33 @@ __device__ __forceinline__ void update_tiles(gdouble *NL, int ldl, gcdouble *X, 
 }
 
 __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
-                                                           const int *lvl_slots,
+                                                           int s0,
                                                            const int *wg_off, int nlvl,
                                                            int step, FactorParams fp) {
   __shared__ double ce1[kBlk], ce2[kBlk];
   __shared__ int ctwo[kBlk];
-  const int li = find_node(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return;
-  NodeDev &N = nodes[lvl_slots[li]];
-  const int local = blockIdx.x - wg_off[li], count = wg_off[li + 1] - wg_off[li];
+  NodeDev &N = nodes[s0 + li];
+  const int local = blockIdx.x - before, count = wg_off[li + 1] - before;
+  const int nsteps = N.nsteps, p = N.p, w = N.w, m = N.m, cend = N.n, nl = N.ldl,
+            nldbak = N.ldbak;
+  double *const nL = N.L, *const nX = N.X;
+  const unsigned long long fail = N.fail;
+  loaded(count, nsteps, p, w, m, cend, nl, nldbak, nL, nX, fail);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (step >= N.nsteps) return;
-  const int p = N.p, w = N.w;
-  if (w == 0) return;
-  const int np = fp.posdef ? w : block_npass(N);
+  if (local >= count || step >= nsteps || w == 0) return;
+  const int np = fp.posdef ? w : block_npass(N, p, w, fail);
   if (local == 0 && tid == 0) N.npass = np;
-  const int a0 = p, K = np, t0 = p + np, cend = N.n, fa = p + np, fb = p + w;
-  const int m = N.m;
+  const int a0 = p, K = np, t0 = p + np, fa = p + np, fb = p + w;
   if (m - t0 <= 0 || cend - t0 <= 0) return;
   const int TI = (m - t0 + kTile - 1) / kTile, TJ = (cend - t0 + kTile - 1) / kTile;
   const int ntiles = TJ * TI - TJ * (TJ - 1) / 2;
   if (np == kBlk) {
-    gdouble *NL = (gdouble *)N.L;
-    gcdouble *X = (gcdouble *)N.X;
-    const int ldl = N.ldl, ldx = N.ldbak;
+    gdouble *NL = (gdouble *)nL;
+    gcdouble *X = (gcdouble *)nX;
+    const int ldl = nl, ldx = nldbak;
     // a run of consecutive tiles each; workgroups go to the eight XCDs in
     // turn, and the runs of one XCD's workgroups are neighbours, so that its
     // L2 holds the operands of few tile columns
@@ -1289,9 +1289,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
 // each trailing index (pmap) and, for each 64-row tile of the parent, the
 // first trailing index whose parent position reaches the tile (ptab).
 constexpr int kMapParts = 8;  // workgroups per front (trailing indices strided over them)
-__global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, int s0,
                                                      const int *child_list) {
-  const NodeDev &P = nodes[lvl_slots[blockIdx.x]];
+  const NodeDev &P = nodes[s0 + blockIdx.x];
   if (P.skip) return;
   const int part = blockIdx.y;
   const int T = (P.m + kGT - 1) / kGT;
@@ -1326,14 +1326,15 @@ __global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, const int *
 // mixed-precision factorization, whose Schur terms then run on FP32 MFMA)
 template <int PART, typename CT>
 __device__ __forceinline__ int gather_tile(
-    NodeDev *nodes, const int *lvl_slots, const int *wg_off, int nlvl,
+    NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
     const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int (&mr)[kGT],
     int (&mc)[kGT]) {
   constexpr bool F32 = sizeof(CT) == 4;
-  const int li = find_node(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return -1;
-  const int s = lvl_slots[li];
+  const int s = s0 + li;
   NodeDev &P = nodes[s];
   // descriptor fields once, into registers (loads below never wait on them)
   const int m = P.m, n = P.n, nd = P.nd, pldl = P.ldl, pldc = P.ldc;
@@ -1346,8 +1347,8 @@ __device__ __forceinline__ int gather_tile(
   const int T = (m + kGT - 1) / kGT;
   // PART 1: the diagonal tile (0, 0); 3: the first tile column's other
   // tiles; 2: the tiles outside the first column; 0: every tile
-  const int local = blockIdx.x - wg_off[li] + (PART == 2 ? T : PART == 3 ? 1 : 0);
-  if (local >= (PART == 1 ? 1 : PART == 3 ? T : T * (T + 1) / 2)) return -1;
+  const int local = blockIdx.x - before + (PART == 2 ? T : PART == 3 ? 1 : 0);
+  if (local >= (PART == 1 ? imin(T, 1) : PART == 3 ? T : T * (T + 1) / 2)) return -1;
   int I, J;
   tile_of(local, T, T, I, J);
   const int r0 = I * kGT, c0 = J * kGT;
@@ -1582,12 +1583,12 @@ __device__ __forceinline__ int gather_tile(
 
 template <int PART, typename CT>
 __global__ __launch_bounds__(kThreads, 4) void k_gather(
-    NodeDev *nodes, const int *lvl_slots, const int *wg_off, int nlvl,
+    NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
     const int *acix, const double *scaling) {
   __shared__ double acc[kGT][kGT + 1];
   __shared__ int mr[kGT], mc[kGT];
-  gather_tile<PART, CT>(nodes, lvl_slots, wg_off, nlvl, child_list, aval, asrc, arow, acix,
+  gather_tile<PART, CT>(nodes, s0, wg_off, nlvl, child_list, aval, asrc, arow, acix,
                         scaling, acc, mr, mc);
 }
 
@@ -1606,18 +1607,20 @@ __device__ inline double *swp_at(double *L, int ldl, int a, int b) {
   return L + (size_t)imin(a, b) * ldl + imax(a, b);
 }
 
-__global__ __launch_bounds__(kThreads) void k_swap(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(kThreads) void k_swap(NodeDev *nodes, int s0,
                                                    const int *wg_off, int nlvl, int step) {
-  const int li = find_node(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return;
-  NodeDev &N = nodes[lvl_slots[li]];
-  if (step >= N.nsteps || N.w == 0) return;
-  const int f0 = N.p + N.npass, pw = N.p + N.w;
-  const int ns = imin(pw - f0, N.q - pw);
-  if (ns <= 0) return;
-  const int u0 = N.q - ns, m = N.m, ldl = N.ldl;
+  NodeDev &N = nodes[s0 + li];
+  const int local = blockIdx.x - before, count = wg_off[li + 1] - before;
+  const int nsteps = N.nsteps, p = N.p, w = N.w, npass = N.npass, q = N.q;
+  loaded(count, nsteps, p, w, npass, q);
+  const int f0 = p + npass, pw = p + w;
+  const int ns = imin(pw - f0, q - pw);
+  if (local >= count || step >= nsteps || w == 0 || ns <= 0) return;
+  const int u0 = q - ns, m = N.m, ldl = N.ldl;
   double *L = N.L;
-  const int local = blockIdx.x - wg_off[li], count = wg_off[li + 1] - wg_off[li];
   const int total = ns * m;
   for (int idx = local * kThreads + threadIdx.x; idx < total; idx += count * kThreads) {
     const int i = idx / m, x = idx - i * m;
@@ -2209,10 +2212,10 @@ __device__ int tpp_front(NodeDev &N, const FactorParams &fp, int nelim, TppShare
 // written here are re-read only after a barrier.
 // ---------------------------------------------------------------------------
 template <int NT>
-__global__ __launch_bounds__(NT) void k_tail(NodeDev *nodes, const int *lvl_slots,
+__global__ __launch_bounds__(NT) void k_tail(NodeDev *nodes, int s0,
                                                    FactorParams fp, int *scratch) {
   __shared__ TppShared<NT> sh;
-  NodeDev &N = nodes[lvl_slots[blockIdx.x]];
+  NodeDev &N = nodes[s0 + blockIdx.x];
   const int tid = threadIdx.x;
   int nelim;
   {
@@ -2447,7 +2450,7 @@ void launch_pack_nodes(hipStream_t st, const NodeDev *nodes, int nn, int *out) {
   if (nn > 0)
     hipLaunchKernelGGL(k_pack_nodes, dim3((nn + 255) / 256), dim3(256), 0, st, nodes, nn, out);
 }
-void launch_gather_first(hipStream_t st, int nwg, NodeDev *nodes, const int *slots,
+void launch_gather_first(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                          const int *wg_off, int nlvl, const int *child_list,
                          const double *aval, const int64_t *asrc, const int *arow,
                          const int *acix, const double *scaling, FactorParams fp) {
@@ -2455,12 +2458,12 @@ void launch_gather_first(hipStream_t st, int nwg, NodeDev *nodes, const int *slo
   if (nwg <= 0) return;
   if (fp.c32)
     hipLaunchKernelGGL((k_diag<kDiagWaves, true, true>), dim3(nwg), dim3(64 * kDiagWaves), 0,
-                       st, nodes, slots, 0, fp, ga);
+                       st, nodes, s0, 0, fp, ga);
   else
     hipLaunchKernelGGL((k_diag<kDiagWaves, true, false>), dim3(nwg), dim3(64 * kDiagWaves), 0,
-                       st, nodes, slots, 0, fp, ga);
+                       st, nodes, s0, 0, fp, ga);
 }
-void launch_gather(hipStream_t st, int part, int nwg, NodeDev *nodes, const int *slots,
+void launch_gather(hipStream_t st, int part, int nwg, NodeDev *nodes, int s0,
                    const int *wg_off, int nlvl, const int *child_list, const double *aval,
                    const int64_t *asrc, const int *arow, const int *acix,
                    const double *scaling, int c32) {
@@ -2471,52 +2474,52 @@ void launch_gather(hipStream_t st, int part, int nwg, NodeDev *nodes, const int 
                   : ((part == 3)   ? k_gather<3, double>
                      : (part == 2) ? k_gather<2, double>
                                    : k_gather<0, double>);
-  hipLaunchKernelGGL(kern, dim3(nwg), dim3(kThreads), 0, st, nodes, slots, wg_off, nlvl,
+  hipLaunchKernelGGL(kern, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off, nlvl,
                      child_list, aval, asrc, arow, acix, scaling);
 }
-void launch_maptab(hipStream_t st, int nlvl, NodeDev *nodes, const int *slots,
+void launch_maptab(hipStream_t st, int nlvl, NodeDev *nodes, int s0,
                    const int *child_list) {
   if (nlvl > 0)
-    hipLaunchKernelGGL(k_maptab, dim3(nlvl, kMapParts), dim3(kThreads), 0, st, nodes, slots,
+    hipLaunchKernelGGL(k_maptab, dim3(nlvl, kMapParts), dim3(kThreads), 0, st, nodes, s0,
                        child_list);
 }
-void launch_tail(hipStream_t st, int nlvl, NodeDev *nodes, const int *slots, FactorParams fp,
+void launch_tail(hipStream_t st, int nlvl, NodeDev *nodes, int s0, FactorParams fp,
                  int *scratch) {
   if (nlvl <= 0) return;
   if (nlvl < kTailWideMaxFronts)
-    hipLaunchKernelGGL(k_tail<kTailWide>, dim3(nlvl), dim3(kTailWide), 0, st, nodes, slots, fp,
+    hipLaunchKernelGGL(k_tail<kTailWide>, dim3(nlvl), dim3(kTailWide), 0, st, nodes, s0, fp,
                        scratch);
   else
-    hipLaunchKernelGGL(k_tail<kTailNarrow>, dim3(nlvl), dim3(kTailNarrow), 0, st, nodes, slots,
+    hipLaunchKernelGGL(k_tail<kTailNarrow>, dim3(nlvl), dim3(kTailNarrow), 0, st, nodes, s0,
                        fp, scratch);
 }
-void launch_diag(hipStream_t st, int nlvl, NodeDev *nodes, const int *slots, int step,
+void launch_diag(hipStream_t st, int nlvl, NodeDev *nodes, int s0, int step,
                  FactorParams fp) {
   if (nlvl > 0)
     hipLaunchKernelGGL((k_diag<kDiagWaves, false, false>), dim3(nlvl), dim3(64 * kDiagWaves),
                        0, st,
-                       nodes, slots, step, fp, GatherArgs{});
+                       nodes, s0, step, fp, GatherArgs{});
 }
-void launch_apply(hipStream_t st, int nwg, NodeDev *nodes, const int *slots,
+void launch_apply(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                   const int *wg_off, int nlvl, int step, FactorParams fp) {
   if (nwg > 0)
-    hipLaunchKernelGGL(k_apply, dim3(nwg), dim3(kThreads), 0, st, nodes, slots, wg_off,
+    hipLaunchKernelGGL(k_apply, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
                        nlvl, step, fp);
 }
-void launch_update(hipStream_t st, int nwg, NodeDev *nodes, const int *slots,
+void launch_update(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                    const int *wg_off, int nlvl, int step, int mode, FactorParams fp) {
   if (nwg <= 0) return;
   if (mode == 0)
-    hipLaunchKernelGGL(k_update_panel, dim3(nwg), dim3(kThreads), 0, st, nodes, slots, wg_off,
+    hipLaunchKernelGGL(k_update_panel, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
                        nlvl, step, fp);
   else
-    hipLaunchKernelGGL(k_update, dim3(nwg), dim3(kThreads), 0, st, nodes, slots, wg_off,
+    hipLaunchKernelGGL(k_update, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
                        nlvl, step, mode, fp);
 }
-void launch_swap(hipStream_t st, int nwg, NodeDev *nodes, const int *slots,
+void launch_swap(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                  const int *wg_off, int nlvl, int step) {
   if (nwg > 0)
-    hipLaunchKernelGGL(k_swap, dim3(nwg), dim3(kThreads), 0, st, nodes, slots, wg_off,
+    hipLaunchKernelGGL(k_swap, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
                        nlvl, step);
 }
 void launch_stats(hipStream_t st, const NodeDev *nodes, int nslots, int *counters,

@@ -29,28 +29,28 @@
 namespace ssids_hip {
 
 // kernel launchers (factor_kernels.hip / solve_kernels.hip)
-void launch_gather(hipStream_t, int, int, NodeDev *, const int *, const int *, int, const int *,
+void launch_gather(hipStream_t, int, int, NodeDev *, int, const int *, int, const int *,
                    const double *, const int64_t *, const int *, const int *, const double *,
                    int);
-void launch_gather_first(hipStream_t, int, NodeDev *, const int *, const int *, int,
+void launch_gather_first(hipStream_t, int, NodeDev *, int, const int *, int,
                          const int *, const double *, const int64_t *, const int *,
                          const int *, const double *, FactorParams);
-void launch_maptab(hipStream_t, int, NodeDev *, const int *, const int *);
-void launch_diag(hipStream_t, int, NodeDev *, const int *, int, FactorParams);
-void launch_apply(hipStream_t, int, NodeDev *, const int *, const int *, int, int,
+void launch_maptab(hipStream_t, int, NodeDev *, int, const int *);
+void launch_diag(hipStream_t, int, NodeDev *, int, int, FactorParams);
+void launch_apply(hipStream_t, int, NodeDev *, int, const int *, int, int,
                   FactorParams);
-void launch_update(hipStream_t, int, NodeDev *, const int *, const int *, int, int, int,
+void launch_update(hipStream_t, int, NodeDev *, int, const int *, int, int, int,
                    FactorParams);
-void launch_swap(hipStream_t, int, NodeDev *, const int *, const int *, int, int);
-void launch_tail(hipStream_t, int, NodeDev *, const int *, FactorParams, int *);
+void launch_swap(hipStream_t, int, NodeDev *, int, const int *, int, int);
+void launch_tail(hipStream_t, int, NodeDev *, int, FactorParams, int *);
 void launch_stats(hipStream_t, const NodeDev *, int, int *, const FactorParams &);
 void launch_level_setup(hipStream_t, NodeDev *, int, int, const int *, int, int, int *, int *);
 void launch_pack_nodes(hipStream_t, const NodeDev *, int, int *);
 void launch_pack_dperm(hipStream_t, const NodeDev *, const int *, const int64_t *, int, double *,
                        int *);
-void launch_fwd_tri(hipStream_t, int, const SolveNode *, const int *, const int *, double *,
+void launch_fwd_tri(hipStream_t, int, const SolveNode *, int, const int *, double *,
                     int, int, double *);
-void launch_fwd_rows(hipStream_t, int, const SolveNode *, const int *, const int *, int,
+void launch_fwd_rows(hipStream_t, int, const SolveNode *, int, const int *, int,
                      const int *, int, double *);
 void launch_big_fwd_lvl(hipStream_t, const SolveNode *, const int *, int, int, const int *,
                         double *, int, int, double *, int *);
@@ -62,7 +62,7 @@ int fwd_rows_per_wg();
 int bwd_rows_per_wg();
 int bwd_cols_per_wg();
 void launch_dsolve(hipStream_t, int, const SolveNode *, double *, int, int, int);
-void launch_bwd(hipStream_t, int, const SolveNode *, const int *, double *, int, int,
+void launch_bwd(hipStream_t, int, const SolveNode *, int, double *, int, int,
                 const int *, const int *, int, double *, int, int);
 
 void launch_residual(hipStream_t, int, const int64_t *, const int *, const int64_t *,
@@ -309,14 +309,13 @@ struct Numeric {
   std::vector<int> nd_seen;               // per slot: most delays seen in a factor
   std::vector<NodeDev> nodes;             // slot-indexed host mirror
   NodeDev *d_nodes = nullptr;
-  int *d_lvl = nullptr;                   // per-level scratch (slots + offsets)
+  int *d_lvl = nullptr;                   // per-level scratch (launch tables)
   size_t d_lvl_cap = 0;
   int *d_counters = nullptr;
   int *d_scratch_n = nullptr;             // n ints (ipos)
   std::vector<std::pair<void *, size_t>> persistent;
   // solve
   SolveNode *d_sn = nullptr;
-  int *d_slots_all = nullptr;             // 0..nnodes-1 (slots in level order)
   // per level: nlvl+1 workgroup offsets of the solve's row kernels (forward:
   // 64-row workgroups, backward: 256-row workgroups), one array
   int *d_gemv_tab = nullptr;
@@ -360,7 +359,6 @@ struct Numeric {
     if (d_counters) (void)hipFree(d_counters);
     if (d_scratch_n) (void)hipFree(d_scratch_n);
     if (d_sn) (void)hipFree(d_sn);
-    if (d_slots_all) (void)hipFree(d_slots_all);
     if (d_gemv_tab) (void)hipFree(d_gemv_tab);
     if (d_bigtab) (void)hipFree(d_bigtab);
     if (d_X) (void)hipFree(d_X);
@@ -857,20 +855,19 @@ static bool factor_static(Numeric &N, const FactorParams &fp, const spral_ssids_
     const int ms = lv.maxsteps;
     int *tab = P.d_tabs + lv.tab_off;
     auto toff = [&](int t) { return (const int *)(tab + (size_t)t * (nl + 1)); };
-    const int *d_slots = N.d_slots_all + s0;
     launch_level_setup(st, N.d_nodes, s0, nl, S.d_child, fp.pivot_tpp, ms, tab, overflow);
-    launch_maptab(st, nl, N.d_nodes, d_slots, S.d_child);
+    launch_maptab(st, nl, N.d_nodes, s0, S.d_child);
     HIPCHK(hipEventRecord(N.ev_level, st));
     HIPCHK(hipStreamWaitEvent(st2, N.ev_level, 0));
     // the first tile column's other tiles on st2, ahead of the rest
-    launch_gather(st2, 3, lv.cap[2 * ms + 5], N.d_nodes, d_slots, toff(2 * ms + 5), nl,
+    launch_gather(st2, 3, lv.cap[2 * ms + 5], N.d_nodes, s0, toff(2 * ms + 5), nl,
                   S.d_child, N.d_aval, S.d_asrc, S.d_arow, S.d_acix, N.d_scal, fp.c32);
     HIPCHK(hipEventRecord(N.ev_first, st2));
     // the diagonal tiles, each with step 0's pivot block
-    launch_gather_first(st, lv.cap[2 * ms + 3], N.d_nodes, d_slots, toff(2 * ms + 3), nl,
+    launch_gather_first(st, lv.cap[2 * ms + 3], N.d_nodes, s0, toff(2 * ms + 3), nl,
                         S.d_child, N.d_aval, S.d_asrc, S.d_arow, S.d_acix, N.d_scal, fp);
     if (opt.timing) tev.emplace_back(timed_event(st2));
-    launch_gather(st2, 2, lv.cap[2 * ms + 4], N.d_nodes, d_slots, toff(2 * ms + 4), nl,
+    launch_gather(st2, 2, lv.cap[2 * ms + 4], N.d_nodes, s0, toff(2 * ms + 4), nl,
                   S.d_child, N.d_aval, S.d_asrc, S.d_arow, S.d_acix, N.d_scal, fp.c32);
     if (opt.timing) tev.emplace_back(timed_event(st2));
     HIPCHK(hipEventRecord(N.ev_rest, st2));
@@ -880,23 +877,23 @@ static bool factor_static(Numeric &N, const FactorParams &fp, const spral_ssids_
       joined = true;
     };
     for (int stp = 0; stp < ms; ++stp) {
-      if (stp > 0) launch_diag(st, nl, N.d_nodes, d_slots, stp, fp);
+      if (stp > 0) launch_diag(st, nl, N.d_nodes, s0, stp, fp);
       // step 0's apply reads the whole first tile column
       if (stp == 0) HIPCHK(hipStreamWaitEvent(st, N.ev_first, 0));
-      launch_apply(st, lv.cap[1 + stp], N.d_nodes, d_slots, toff(1 + stp), nl, stp, fp);
+      launch_apply(st, lv.cap[1 + stp], N.d_nodes, s0, toff(1 + stp), nl, stp, fp);
       // one step (every n <= 64): the update stays inside the first tile
       // column too; with more steps it reaches the later columns
       if (ms > 1) join();
-      launch_update(st, lv.cap[ms + 2 + stp], N.d_nodes, d_slots, toff(ms + 2 + stp), nl, stp,
+      launch_update(st, lv.cap[ms + 2 + stp], N.d_nodes, s0, toff(ms + 2 + stp), nl, stp,
                     0, fp);
       // (the last step leaves no unprocessed candidate to swap with)
       if (stp + 1 < ms)
-        launch_swap(st, lv.cap[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp);
+        launch_swap(st, lv.cap[ms + 1], N.d_nodes, s0, toff(ms + 1), nl, stp);
     }
     join();
-    launch_tail(st, nl, N.d_nodes, d_slots, fp, N.d_scratch_n);
+    launch_tail(st, nl, N.d_nodes, s0, fp, N.d_scratch_n);
     if (lv.cap[2 * ms + 2] > 0)
-      launch_update(st, lv.cap[2 * ms + 2], N.d_nodes, d_slots, toff(2 * ms + 2), nl, 0, 1, fp);
+      launch_update(st, lv.cap[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1, fp);
   }
   launch_pack_nodes(st, N.d_nodes, nn, P.d_pack);
   };
@@ -1019,11 +1016,10 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
     }
     HIPCHK(hipMemcpyAsync(N.d_nodes + s0, N.nodes.data() + s0, nl * sizeof(NodeDev),
                           hipMemcpyHostToDevice, st));
-    // per-level launch tables (exact sizes): slots | tables of level_table_count
+    // per-level launch tables (exact sizes) of level_table_count
     const int ntab = level_tables(maxsteps);
     std::vector<int> tab;
-    tab.reserve(nl + (size_t)ntab * (nl + 1));
-    for (int sl = s0; sl < s1; ++sl) tab.push_back(sl);
+    tab.reserve((size_t)ntab * (nl + 1));
     std::vector<int> tot(ntab, 0);
     for (int t = 0; t < ntab; ++t) {
       int acc = 0;
@@ -1038,25 +1034,24 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
     ensure_lvl(N, tab.size());
     HIPCHK(hipMemcpyAsync(N.d_lvl, tab.data(), tab.size() * sizeof(int),
                           hipMemcpyHostToDevice, st));
-    const int *d_slots = N.d_lvl;
-    auto toff = [&](int t) { return (const int *)(N.d_lvl + nl + (size_t)t * (nl + 1)); };
+    auto toff = [&](int t) { return (const int *)(N.d_lvl + (size_t)t * (nl + 1)); };
     const int ms = maxsteps;
-    launch_maptab(st, nl, N.d_nodes, d_slots, S.d_child);
+    launch_maptab(st, nl, N.d_nodes, s0, S.d_child);
     if (opt.timing) tev.emplace_back(timed_event(st));
-    launch_gather(st, 0, tot[0], N.d_nodes, d_slots, toff(0), nl, S.d_child, N.d_aval,
+    launch_gather(st, 0, tot[0], N.d_nodes, s0, toff(0), nl, S.d_child, N.d_aval,
                   S.d_asrc, S.d_arow, S.d_acix, N.d_scal, fp.c32);
     if (opt.timing) tev.emplace_back(timed_event(st));
     for (int stp = 0; stp < ms; ++stp) {
-      launch_diag(st, nl, N.d_nodes, d_slots, stp, fp);
-      launch_apply(st, tot[1 + stp], N.d_nodes, d_slots, toff(1 + stp), nl, stp, fp);
-      launch_update(st, tot[ms + 2 + stp], N.d_nodes, d_slots, toff(ms + 2 + stp), nl, stp, 0,
+      launch_diag(st, nl, N.d_nodes, s0, stp, fp);
+      launch_apply(st, tot[1 + stp], N.d_nodes, s0, toff(1 + stp), nl, stp, fp);
+      launch_update(st, tot[ms + 2 + stp], N.d_nodes, s0, toff(ms + 2 + stp), nl, stp, 0,
                     fp);
       if (stp + 1 < ms)
-        launch_swap(st, tot[ms + 1], N.d_nodes, d_slots, toff(ms + 1), nl, stp);
+        launch_swap(st, tot[ms + 1], N.d_nodes, s0, toff(ms + 1), nl, stp);
     }
-    launch_tail(st, nl, N.d_nodes, d_slots, fp, N.d_scratch_n);
+    launch_tail(st, nl, N.d_nodes, s0, fp, N.d_scratch_n);
     if (tot[2 * ms + 2] > 0)
-      launch_update(st, tot[2 * ms + 2], N.d_nodes, d_slots, toff(2 * ms + 2), nl, 0, 1, fp);
+      launch_update(st, tot[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1, fp);
     HIPCHK(hipGetLastError());
     // read back the level's results (nelim, flag)
     std::vector<NodeDev> back(nl);
@@ -1136,13 +1131,6 @@ static void build_solve_tables(Numeric &N) {
     Q.ctab = D.ctab;
   }
   if (!N.d_sn) HIPCHK(hipMalloc(&N.d_sn, std::max(nn, 1) * sizeof(SolveNode)));
-  if (!N.d_slots_all) {
-    std::vector<int> iota(std::max(nn, 1));
-    for (int i = 0; i < nn; ++i) iota[i] = i;
-    HIPCHK(hipMalloc(&N.d_slots_all, iota.size() * sizeof(int)));
-    copy_now(N.d_slots_all, iota.data(), iota.size() * sizeof(int),
-                     hipMemcpyHostToDevice, N.stream);
-  }
   // solve row-workgroup tables (depend on nelim): every front gets at least
   // one, which in the backward solve also reduces and solves the triangle
   {
@@ -1281,13 +1269,6 @@ static void factor_impl(Numeric &N, const double *d_aval, const double *d_scalin
   if (!N.d_nodes) HIPCHK(hipMalloc(&N.d_nodes, std::max(nn, 1) * sizeof(NodeDev)));
   if (!N.d_counters) HIPCHK(hipMalloc(&N.d_counters, 16 * sizeof(int)));
   if (!N.d_scratch_n) HIPCHK(hipMalloc(&N.d_scratch_n, std::max(S.n, 1) * sizeof(int)));
-  if (!N.d_slots_all) {
-    std::vector<int> iota(std::max(nn, 1));
-    for (int i = 0; i < nn; ++i) iota[i] = i;
-    HIPCHK(hipMalloc(&N.d_slots_all, iota.size() * sizeof(int)));
-    copy_now(N.d_slots_all, iota.data(), iota.size() * sizeof(int),
-                     hipMemcpyHostToDevice, N.stream);
-  }
   HIPCHK(hipMemsetAsync(N.d_counters, 0, 16 * sizeof(int), st));
   std::vector<hipEvent_t> tev;  // pairs around the gather launches
   hipEvent_t ev0, ev1;
@@ -1438,8 +1419,6 @@ static void solve_launch(Numeric &N, int job, int nrhs, double *d_x, int ldx, hi
   // 342-343): the diagonal solve alone is a no-op, diag + bwd is bwd
   if (N.posdef && job == 2) return;
   if (N.posdef && job == 4) job = 3;
-  // the slot list of all levels is simply 0..nnodes-1 in level order
-  const int *slots = N.d_slots_all;
   bool fwd = (job == 0 || job == 1), bwd = (job == 0 || job == 3 || job == 4);
   bool diag = (job == 0 || job == 2 || job == 4);
   // positive definite: L_chol = L D^{1/2}, so the forward (job 1) and
@@ -1451,10 +1430,10 @@ static void solve_launch(Numeric &N, int job, int nrhs, double *d_x, int ldx, hi
     for (int L = 0; L < nlev; ++L) {
       const int nl = S.lvl_ptr[L + 1] - S.lvl_ptr[L], nbig = (int)N.big_of_level[L].size();
       if (nl > nbig)
-        launch_fwd_tri(st, nl, N.d_sn, slots + S.lvl_ptr[L], S.d_child, d_x, ldx, nrhs, ws);
+        launch_fwd_tri(st, nl, N.d_sn, S.lvl_ptr[L], S.d_child, d_x, ldx, nrhs, ws);
       launch_big_fwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], nbig, N.big_blocks[L],
                          S.d_child, d_x, ldx, nrhs, ws, sync);
-      launch_fwd_rows(st, nl, N.d_sn, slots + S.lvl_ptr[L], S.d_child, nrhs,
+      launch_fwd_rows(st, nl, N.d_sn, S.lvl_ptr[L], S.d_child, nrhs,
                       N.d_gemv_tab + N.gemv_tab_off[L], N.gemv_total[L], ws);
     }
   // with a backward solve after it, D^{-1} is applied per front inside the
@@ -1466,7 +1445,7 @@ static void solve_launch(Numeric &N, int job, int nrhs, double *d_x, int ldx, hi
   if (bwd)
     for (int L = nlev - 1; L >= 0; --L) {
       const int nl = S.lvl_ptr[L + 1] - S.lvl_ptr[L], nbig = (int)N.big_of_level[L].size();
-      launch_bwd(st, nl, N.d_sn, slots + S.lvl_ptr[L], d_x, ldx, nrhs,
+      launch_bwd(st, nl, N.d_sn, S.lvl_ptr[L], d_x, ldx, nrhs,
                  N.d_gemv_tab + N.bwd_tab_off[L], N.d_gemv_tab + N.bwdc_tab_off[L],
                  N.bwdc_total[L], ws, dfuse, nl - nbig);
       launch_big_bwd_lvl(st, N.d_sn, N.d_bigtab + N.bigtab_off[L], nbig, N.big_blocks[L], d_x,

@@ -52,10 +52,6 @@ constexpr int kGroups = kThreads / kRows;  // column groups (one wave each)
 constexpr int kBigTri = 256;
 constexpr int kTriCap = 1024;  // fully-summed positions gathered in LDS
 
-__device__ inline int find_node_s(const int *wg_off, int nlvl, int b) {
-  return table_find(wg_off, nlvl, b);
-}
-
 // FP64 MFMA accumulators of the multi-right-hand-side products
 typedef double mr_acc_t __attribute__((ext_vector_type(4)));
 // independent accumulators per output (4-position step u goes to u % kMrSplit,
@@ -185,14 +181,14 @@ constexpr int kChildBatch = 4;
 // by wave, so every position is summed in a fixed order), then the triangle
 // X[0:ne] <- L11^{-1} X[0:ne] when ne <= kBigTri.
 template <int NR>
-__global__ __launch_bounds__(kThreads, 2) void k_fwd_tri(const SolveNode *sn, const int *slots,
+__global__ __launch_bounds__(kThreads, 2) void k_fwd_tri(const SolveNode *sn, int s0,
                                                       const int *child_list, double *x,
                                                       int ldx, int nrhs, double *ws) {
   constexpr int kCap = (NR == 1) ? kTriCap : kBigTri, kLdx = kCap + 2;
   __shared__ double xs[NR][kLdx];
   __shared__ double lb[kBlk][kBlk + 1];
   __shared__ int nchunk[kGroups];
-  const SolveNode &P = sn[slots[blockIdx.x]];
+  const SolveNode &P = sn[s0 + blockIdx.x];
   const double *PL = P.L;
   gcint *Pperm = (gcint *)P.perm;
   gcint *Pipos = (gcint *)P.ipos;
@@ -368,16 +364,18 @@ __global__ __launch_bounds__(kThreads, 2) void k_fwd_tri(const SolveNode *sn, co
 // waves' sums are added in wave order.  L is read once, in whole 512-byte
 // column pieces, the next 64 columns under way during the current ones.
 template <int NR>
-__global__ __launch_bounds__(kThreads, NR == 1 ? 4 : 2) void k_fwd_rows(const SolveNode *sn, const int *slots,
+__global__ __launch_bounds__(kThreads, NR == 1 ? 4 : 2) void k_fwd_rows(const SolveNode *sn, int s0,
                                                        const int *child_list,
                                                        const int *wg_off, int nlvl, int nrhs,
                                                        double *ws) {
   __shared__ double xs[NR][kRows];
   __shared__ double red[kGroups][NR][kRows + 2];
-  const int li = find_node_s(wg_off, nlvl, blockIdx.x);
-  const SolveNode &P = sn[slots[li]];
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
+  if (li < 0) return;
+  const SolveNode &P = sn[s0 + li];
   const int ne = P.nelim, m = P.m;
-  const int r0 = ne + (blockIdx.x - wg_off[li]) * kRows, r1 = imin(m, r0 + kRows);
+  const int r0 = ne + (blockIdx.x - before) * kRows, r1 = imin(m, r0 + kRows);
   if (r0 >= r1) return;  // front without rows below
   const double *PL = P.L;
   gcint *Pctab = (gcint *)P.ctab;
@@ -541,21 +539,22 @@ __global__ void k_dsolve(const SolveNode *sn, int nslots, double *x, int ldx, in
 constexpr int kBwdCols = 64;
 typedef double double2_u __attribute__((ext_vector_type(2), aligned(8)));
 __global__ __launch_bounds__(kThreads, 2) void k_bwd_rows(const SolveNode *sn,
-                                                             const int *slots,
+                                                             int s0,
                                                              const int *wg_off, int nlvl,
                                                              const double *x, int ldx, int nrhs,
                                                              double *ws) {
   constexpr int kSteps = 16;  // rows of a lane
   __shared__ double red[kGroups][kRhsGroup][kBwdCols + 2];
-  const int li = find_node_s(wg_off, nlvl, blockIdx.x);
+  int before;
+  const int li = front_of(wg_off, nlvl, blockIdx.x, before);
   if (li < 0) return;
-  const SolveNode &P = sn[slots[li]];
+  const SolveNode &P = sn[s0 + li];
   gcint *Pperm = (gcint *)P.perm;
   gcint *Prows = (gcint *)P.rows;
   gdouble *part = (gdouble *)solve_P(ws, P, nrhs);  // count x nrhs x ne
   const int ldl = P.ldl, m = P.m, n = P.n, nd = P.nd, ne = P.nelim;
   const int nchunk = idiv_up(imax(ne, 1), kBwdCols);
-  const int local_all = blockIdx.x - wg_off[li];
+  const int local_all = blockIdx.x - before;
   const int local = local_all / nchunk, chunk = local_all - local * nchunk;
   const int jbeg = chunk * kBwdCols, jend = imin(ne, jbeg + kBwdCols);
   const int r0 = ne + local * kThreads, r1 = imin(m, r0 + kThreads);
@@ -651,14 +650,14 @@ __device__ inline double part_sum(gcdouble *p, size_t stride, int count) {
 // right-hand sides: X[j] = x[perm[j]] - sum of the row workgroups' partials, then the triangle
 // L11^T X = X, 64-column blocks from the last, and x[perm[j]] = X[j].
 template <int NR>
-__global__ __launch_bounds__(kThreads, NR == 1 ? 3 : 2) void k_bwd_tri(const SolveNode *sn, const int *slots,
+__global__ __launch_bounds__(kThreads, NR == 1 ? 3 : 2) void k_bwd_tri(const SolveNode *sn, int s0,
                                                       const int *wg_off, double *x, int ldx,
                                                       int nrhs, double *ws, int dfuse) {
   constexpr int kLdx = kBigTri + 2;
   __shared__ double xt[NR][kLdx];
   __shared__ double lb[kBlk][kBlk + 1];
   const int li = blockIdx.x;
-  const SolveNode &P = sn[slots[li]];
+  const SolveNode &P = sn[s0 + li];
   const double *PL = P.L;
   gcdouble *Pd = (gcdouble *)P.D;
   gcint *Pperm = (gcint *)P.perm;
@@ -817,7 +816,8 @@ __global__ __launch_bounds__(kThreads) void k_big_fwd_init(const SolveNode *sn, 
                                                            const double *x, int ldx, int nrhs,
                                                            double *ws) {
   __shared__ double xs[kInitRhs][kBlk];
-  const int li = table_find(boff, nbig, blockIdx.x);
+  int before;  // (the grid is the table's total)
+  const int li = front_of(boff, nbig, blockIdx.x, before);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
   gcint *Pipos = (gcint *)P.ipos;
@@ -830,7 +830,7 @@ __global__ __launch_bounds__(kThreads) void k_big_fwd_init(const SolveNode *sn, 
     const int nr = imin(kInitRhs, nrhs - rc);
     double *X = solve_X(ws, P, nrhs) + (size_t)rc * m;
     double *Y = solve_P(ws, P, nrhs) + (size_t)rc * ne;
-    for (int t = blockIdx.x - boff[li]; t < Tn; t += nb) {
+    for (int t = blockIdx.x - before; t < Tn; t += nb) {
       const int pre0 = 64 * t, pp = pre0 + lane;
       int pos = -1;
       if (pp < n) {
@@ -880,11 +880,12 @@ __global__ __launch_bounds__(kThreads) void k_big_bwd_init(const SolveNode *sn, 
                                                            const int *bslot, int nbig,
                                                            const double *x, int ldx, int nrhs,
                                                            double *ws, int dfuse) {
-  const int li = table_find(boff, nbig, blockIdx.x);
+  int before;  // (the grid is the table's total)
+  const int li = front_of(boff, nbig, blockIdx.x, before);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
   const int m = P.m, ne = P.nelim, count = idiv_up(m - ne, kThreads);
-  const int j = (blockIdx.x - boff[li]) * kBlk + (threadIdx.x & 63);
+  const int j = (blockIdx.x - before) * kBlk + (threadIdx.x & 63);
   if (j >= ne) return;
   gcint *Pperm = (gcint *)P.perm;
   double *PX = solve_X(ws, P, nrhs), *PY = solve_P(ws, P, nrhs);
@@ -964,7 +965,8 @@ __global__ __launch_bounds__(kThreads) void k_big_fwd_lvl(const SolveNode *sn, c
                                                           int nrhs, int rg, double *ws, int *sync) {
   __shared__ double red[kRhsGroup][kBlk];
   __shared__ int s_b;
-  const int li = table_find(boff, nbig, blockIdx.x);
+  int before;  // (the grid is the table's total)
+  const int li = front_of(boff, nbig, blockIdx.x, before);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1030,7 +1032,8 @@ __global__ __launch_bounds__(kThreads) void k_big_bwd_lvl(const SolveNode *sn, c
   __shared__ double lb[kBlk][kBlk + 1];
   __shared__ double red[kRhsGroup][kBlk];
   __shared__ int s_b;
-  const int li = table_find(boff, nbig, blockIdx.x);
+  int before;  // (the grid is the table's total)
+  const int li = front_of(boff, nbig, blockIdx.x, before);
   if (li < 0) return;
   const SolveNode &P = sn[bslot[li]];
   const int ne = P.nelim, nb = idiv_up(ne, kBlk);
@@ -1154,31 +1157,31 @@ void launch_big_sync_clear(hipStream_t st, int *sync, int n) {
     hipLaunchKernelGGL(k_big_sync_clear, dim3((n + 255) / 256), dim3(256), 0, st, sync, n);
 }
 
-void launch_fwd_tri(hipStream_t st, int nlvl, const SolveNode *sn, const int *slots,
+void launch_fwd_tri(hipStream_t st, int nlvl, const SolveNode *sn, int s0,
                     const int *child_list, double *x, int ldx, int nrhs, double *ws) {
   if (nlvl <= 0) return;
   if (nrhs == 1)
-    hipLaunchKernelGGL(k_fwd_tri<1>, dim3(nlvl), dim3(kThreads), 0, st, sn, slots, child_list, x,
+    hipLaunchKernelGGL(k_fwd_tri<1>, dim3(nlvl), dim3(kThreads), 0, st, sn, s0, child_list, x,
                        ldx, nrhs, ws);
   else if (rhs_few(nlvl, nrhs))
     hipLaunchKernelGGL(k_fwd_tri<kRhsFew>, dim3(nlvl, rhs_groups(nrhs, kRhsFew)),
-                       dim3(kThreads), 0, st, sn, slots, child_list, x, ldx, nrhs, ws);
+                       dim3(kThreads), 0, st, sn, s0, child_list, x, ldx, nrhs, ws);
   else
     hipLaunchKernelGGL(k_fwd_tri<kRhsGroup>, dim3(nlvl, rhs_groups(nrhs, kRhsGroup)),
-                       dim3(kThreads), 0, st, sn, slots, child_list, x, ldx, nrhs, ws);
+                       dim3(kThreads), 0, st, sn, s0, child_list, x, ldx, nrhs, ws);
 }
-void launch_fwd_rows(hipStream_t st, int nlvl, const SolveNode *sn, const int *slots,
+void launch_fwd_rows(hipStream_t st, int nlvl, const SolveNode *sn, int s0,
                      const int *child_list, int nrhs, const int *wg_off, int nwg, double *ws) {
   if (nlvl <= 0 || nwg <= 0) return;
   if (nrhs == 1)
-    hipLaunchKernelGGL(k_fwd_rows<1>, dim3(nwg), dim3(kThreads), 0, st, sn, slots, child_list,
+    hipLaunchKernelGGL(k_fwd_rows<1>, dim3(nwg), dim3(kThreads), 0, st, sn, s0, child_list,
                        wg_off, nlvl, nrhs, ws);
   else if (rhs_few(nwg, nrhs))
     hipLaunchKernelGGL(k_fwd_rows<kRhsFew>, dim3(nwg, rhs_groups(nrhs, kRhsFew)),
-                       dim3(kThreads), 0, st, sn, slots, child_list, wg_off, nlvl, nrhs, ws);
+                       dim3(kThreads), 0, st, sn, s0, child_list, wg_off, nlvl, nrhs, ws);
   else
     hipLaunchKernelGGL(k_fwd_rows<kRhsGroup>, dim3(nwg, rhs_groups(nrhs, kRhsGroup)),
-                       dim3(kThreads), 0, st, sn, slots, child_list, wg_off, nlvl, nrhs, ws);
+                       dim3(kThreads), 0, st, sn, s0, child_list, wg_off, nlvl, nrhs, ws);
 }
 void launch_dsolve(hipStream_t st, int nslots, const SolveNode *sn, double *x, int ldx,
                    int nrhs, int half) {
@@ -1188,23 +1191,23 @@ void launch_dsolve(hipStream_t st, int nslots, const SolveNode *sn, double *x, i
 }
 // rows_off: the level's 256-row workgroup table (per front); chunk_off /
 // nwg: the row workgroups x column chunks table of k_bwd_rows and its total
-void launch_bwd(hipStream_t st, int nlvl, const SolveNode *sn, const int *slots, double *x,
+void launch_bwd(hipStream_t st, int nlvl, const SolveNode *sn, int s0, double *x,
                 int ldx, int nrhs, const int *rows_off, const int *chunk_off, int nwg,
                 double *ws, int dfuse, int ntri) {
   if (nlvl <= 0) return;
   if (nwg > 0)
     hipLaunchKernelGGL(k_bwd_rows, dim3(nwg, rhs_groups(nrhs, kRhsGroup)), dim3(kThreads), 0,
-                       st, sn, slots, chunk_off, nlvl, x, ldx, nrhs, ws);
+                       st, sn, s0, chunk_off, nlvl, x, ldx, nrhs, ws);
   if (ntri <= 0) return;  // big fronts only
   if (nrhs == 1)
-    hipLaunchKernelGGL(k_bwd_tri<1>, dim3(nlvl), dim3(kThreads), 0, st, sn, slots, rows_off, x,
+    hipLaunchKernelGGL(k_bwd_tri<1>, dim3(nlvl), dim3(kThreads), 0, st, sn, s0, rows_off, x,
                        ldx, nrhs, ws, dfuse);
   else if (rhs_few(nlvl, nrhs))
     hipLaunchKernelGGL(k_bwd_tri<kRhsFew>, dim3(nlvl, rhs_groups(nrhs, kRhsFew)),
-                       dim3(kThreads), 0, st, sn, slots, rows_off, x, ldx, nrhs, ws, dfuse);
+                       dim3(kThreads), 0, st, sn, s0, rows_off, x, ldx, nrhs, ws, dfuse);
   else
     hipLaunchKernelGGL(k_bwd_tri<kRhsGroup>, dim3(nlvl, rhs_groups(nrhs, kRhsGroup)),
-                       dim3(kThreads), 0, st, sn, slots, rows_off, x, ldx, nrhs, ws, dfuse);
+                       dim3(kThreads), 0, st, sn, s0, rows_off, x, ldx, nrhs, ws, dfuse);
 }
 
 }  // namespace ssids_hip
