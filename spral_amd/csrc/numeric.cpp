@@ -113,7 +113,11 @@ static hipStream_t thread_stream() {
 // ---------------------------------------------------------------------------
 // Device memory pool: large chunks, best-fit free blocks (indexed by size, so
 // an allocation is O(log blocks) however many fronts a batch places) with
-// coalescing on release.
+// coalescing on release.  A chunk is as large as all before it together, at
+// least 1 MiB and at most 1 GiB, and the first as large as `reserve` said: the
+// driver clears what it maps, so a 1 GiB chunk under a system that uses 20 MB
+// cost a loop of new handles 20 ms a pass (1.8 s at worst) where the
+// factorization and the solve take 3.
 // ---------------------------------------------------------------------------
 class Pool {
  public:
@@ -134,12 +138,13 @@ class Pool {
       peak_ = std::max(peak_, used_);
       return (char *)c.base + off;
     }
-    size_t csz = std::max(bytes, chunk_min_);
+    const size_t csz = std::max(bytes, std::clamp(std::max(total_, reserve_), kChunkLo, kChunkHi));
     Chunk c;
     HIPCHK(hipMalloc(&c.base, csz));
     c.size = csz;
     if (csz > bytes) c.put(bytes, csz - bytes);
     chunks_.push_back(std::move(c));
+    total_ += csz;
     used_ += bytes;
     peak_ = std::max(peak_, used_);
     return chunks_.back().base;
@@ -174,7 +179,7 @@ class Pool {
       }
     }
   }
-  void set_chunk_min(size_t b) { chunk_min_ = b; }
+  void reserve(size_t b) { reserve_ = (b + 4095) & ~size_t(4095); }
   size_t peak() const { return peak_; }
 
  private:
@@ -189,7 +194,8 @@ class Pool {
     }
   };
   std::vector<Chunk> chunks_;
-  size_t chunk_min_ = size_t(1) << 30;
+  static constexpr size_t kChunkLo = size_t(1) << 20, kChunkHi = size_t(1) << 30;
+  size_t reserve_ = 0, total_ = 0;
   size_t used_ = 0, peak_ = 0;
 };
 
@@ -687,6 +693,30 @@ static size_t arena_place(std::vector<ArenaBlock> &b) {
   return arena;
 }
 
+// Twice what a plan without delays takes from the pool (every front's kept
+// buffers, and the level whose fronts' and children's transient blocks are
+// largest), which leaves room for delays and for gaps between blocks: a second
+// chunk costs 0.3 ms.
+static size_t plan_estimate(const Numeric &N) {
+  const Symbolic &S = *N.symb;
+  size_t kept = 0, trans = 0;
+  for (size_t L = 0; L + 1 < S.lvl_ptr.size(); ++L) {
+    size_t lev = 0;
+    for (int sl = S.lvl_ptr[L]; sl < S.lvl_ptr[L + 1]; ++sl) {
+      const int i = S.node_of[sl];
+      const size_t m = S.sm[i], n = S.sn[i], ld = (m + 15) & ~size_t(15);
+      kept += ld * n * sizeof(double) + 64 * n + 4 * m + 2048;
+      lev += (2 * m + 2 * kBlk) * kBlk * sizeof(double) + ld * m * sizeof(double);
+      for (int c : S.children[i]) {
+        const size_t k = S.sm[c] - S.sn[c];
+        lev += k * (k + S.sn[c]) * sizeof(double);
+      }
+    }
+    trans = std::max(trans, lev);
+  }
+  return 2 * (kept + trans);
+}
+
 // Place every front for a delay capacity of
 //   ndcap = seen + ceil((multiplier - 1) (sn + seen)),
 // at most the children's fully-summed columns and at most what fits in the
@@ -700,6 +730,7 @@ static void plan_build(Numeric &N, int pivot_tpp, double multiplier) {
   N.persistent.clear();
   const int nn = S.nnodes, nlev = (int)S.lvl_ptr.size() - 1;
   if ((int)N.nd_seen.size() != nn) N.nd_seen.assign(nn, 0);
+  N.pool.reserve(plan_estimate(N));
   const double slack = std::max(0.0, multiplier - 1.0);
   P.pivot_tpp = pivot_tpp;
   P.c32 = N.c32;
