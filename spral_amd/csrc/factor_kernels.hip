@@ -1317,6 +1317,36 @@ __global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, int s0,
   }
 }
 
+// Tile of a front's workgroup `local` of `count`, for the lower tiles of a
+// T x T front from tile column `jfirst` on.  Workgroups go to the eight XCDs in
+// turn, each with an L2 of its own, so workgroups 8 apart take neighbouring
+// tiles: of every 1,024 (what runs at once) an XCD takes 128 in sequence, in
+// strips of eight tile columns traversed by rows.  The 128 tiles read some 16
+// + 8 rows of 64 of the children's L21 and L21 D; down the columns and across
+// the XCDs it was up to T + 16.
+constexpr int kXcd = 8, kXcdRun = 128, kStrip = 8;
+__device__ inline void gather_place(int local, int count, int T, int jfirst, int &I, int &J) {
+  const int base = local & ~(kXcd * kXcdRun - 1), l = local - base;
+  const int rem = imin(count - base, kXcd * kXcdRun);
+  const int x = l & (kXcd - 1), q = rem / kXcd, r = rem & (kXcd - 1);
+  const int at = base + x * q + imin(x, r) + l / kXcd;
+  auto first = [&](int j) { return j * T - j * (j - 1) / 2; };  // tiles before column j
+  const int start = first(jfirst);
+  tile_of(start + at, T, T, I, J);
+  const int c = J - ((J - jfirst) & (kStrip - 1)), w = imin(kStrip, T - c);
+  int in = start + at - first(c);
+  const int tri = w * (w + 1) / 2;
+  if (in < tri) {
+    I = c;
+    while (in > I - c) in -= I++ - c + 1;
+    J = c + in;
+  } else {
+    in -= tri;
+    I = c + w + in / w;
+    J = c + in % w;
+  }
+}
+
 // PART 0: every tile of the level's fronts; 1: the first tile column only
 // (the pivot block and the rows below it); 2: the remaining tiles
 // Returns the front's slot when this workgroup built the front's first
@@ -1347,10 +1377,19 @@ __device__ __forceinline__ int gather_tile(
   const int T = (m + kGT - 1) / kGT;
   // PART 1: the diagonal tile (0, 0); 3: the first tile column's other
   // tiles; 2: the tiles outside the first column; 0: every tile
-  const int local = blockIdx.x - before + (PART == 2 ? T : PART == 3 ? 1 : 0);
-  if (local >= (PART == 1 ? imin(T, 1) : PART == 3 ? T : T * (T + 1) / 2)) return -1;
+  const int local = blockIdx.x - before;
+  const int count = PART == 1 ? imin(T, 1)
+                    : PART == 3 ? T - 1
+                    : PART == 2 ? T * (T - 1) / 2
+                                : T * (T + 1) / 2;
+  if (local >= count) return -1;
   int I, J;
-  tile_of(local, T, T, I, J);
+  if constexpr (PART == 1 || PART == 3) {
+    I = local + (PART == 3 ? 1 : 0);
+    J = 0;
+  } else {
+    gather_place(local, count, T, PART == 2 ? 1 : 0, I, J);
+  }
   const int r0 = I * kGT, c0 = J * kGT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int idx = tid; idx < kGT * kGT; idx += kThreads) acc[idx % kGT][idx / kGT] = 0.0;
