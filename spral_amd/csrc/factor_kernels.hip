@@ -5,9 +5,9 @@
 // per-level prefix array of workgroup counts (wg_off).
 //
 //  k_gather     gather assembly: a workgroup builds a 64x64 tile of one parent
-//               front in LDS from its children (children in order =>
-//               deterministic sums) through LDS-staged child->parent maps,
-//               computing the children's Schur complements on MFMA on the way.
+//               front in registers from its children (children in order =>
+//               deterministic sums) through maps in LDS, computing the
+//               children's Schur complements on MFMA on the way.
 //  k_diag       one workgroup per front: factor the w<=64 column diagonal
 //               block with complete pivoting (1x1/2x2) in registers
 //               (pivot rules of src/ssids/cpu/kernels/block_ldlt.hxx:213-414).
@@ -296,13 +296,13 @@ __device__ __forceinline__ void block_inverse(const double (&mi)[kBlk][kBlk + 1]
 }
 
 constexpr int kGT = 64;  // gather tile edge
+constexpr int kGatherInv = 3 * 2 * kGT;  // ints of LDS for its maps
 
 template <int PART, typename CT>
 __device__ __forceinline__ int gather_tile(
     NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
-    const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int (&mr)[kGT],
-    int (&mc)[kGT]);
+    const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int *inv);
 
 struct GatherArgs {  // the level's gather inputs (a pivot launch that assembles)
   const int *wg_off;
@@ -343,10 +343,11 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, int s0,
   if constexpr (FIRST) {
     static_assert(64 * NW == kThreads, "one workgroup shape for both phases");
     static_assert(kGT == kBlk, "the gather tile is the pivot block's staging array");
-    // the tile's LDS is the pivot block's own (t, lp, inv_lp), used in turn
+    // the tile's LDS is the pivot block's own (t, mi), used in turn
+    static_assert(sizeof(mi) >= kGatherInv * sizeof(int), "mi holds the gather's maps");
     typedef typename std::conditional<C32, float, double>::type CT;
     s = gather_tile<1, CT>(nodes, s0, ga.wg_off, ga.nlvl, ga.child_list, ga.aval,
-                           ga.asrc, ga.arow, ga.acix, ga.scaling, t, lp, inv_lp);
+                           ga.asrc, ga.arow, ga.acix, ga.scaling, t, (int *)mi);
     if (s < 0) return;
     __syncthreads();  // the block's stores are visible to the whole workgroup
   } else {
@@ -1276,14 +1277,24 @@ __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
 // ---------------------------------------------------------------------------
 // Gather assembly of one level (replaces zero + scatter + extend-add + the
 // Schur update of the children's contribution blocks).  A workgroup owns a
-// 64x64 tile of one parent front and builds it in LDS:
+// 64x64 tile of one parent front and builds it in registers:
 //   for each child in order, the child's trailing index ranges that map into
-//   the tile come from the k_maptab tables and their parent positions are
-//   staged in LDS; failed (delayed) columns are copied from the child panel;
-//   contribution columns are added as C_c (read down its columns) minus
+//   the tile come from the k_maptab tables, and the tile's rows and columns
+//   look up their trailing index in LDS; failed (delayed) columns are copied
+//   from the child panel; contribution columns are added as C_c minus
 //   L21 (D L21)^T on MFMA (K = the child's nelim; operands straight from
-//   global memory in the fragment layout), both through the maps;
-//   then the tile's A entries are added and the tile is stored once.
+//   global memory in the fragment layout), both loaded by the tile's own
+//   rows and columns;
+//   then the tile's A entries are added (through LDS) and it is stored once.
+// The tile stays in the MFMA's registers from the first child to the store.
+// Built in LDS, it took three barriers a child and scattered adds: 32^3 27-point
+// KKT (150 levels of one front with a block of 64 pivots, where the gather
+// streams the contribution block) 77.9 -> 74.5 ms.  What bounds it there is the
+// L1's address path (busy 72% of the time), not memory (2.1 TB/s); in FP64 with
+// many pivots it is the matrix cores (half the time busy, the rest waits for
+// operands).  FP64 needs 166 registers, three workgroups a CU (four spill 25
+// registers: 12.4 against 10.7 ms of a 64^3 factorization's gathers); FP32 fits
+// four.  Three or four steps a buffer are slower (11.4 and 12.5 ms).
 // ---------------------------------------------------------------------------
 // Per level, for every child of the level's fronts: the parent position of
 // each trailing index (pmap) and, for each 64-row tile of the parent, the
@@ -1358,8 +1369,7 @@ template <int PART, typename CT>
 __device__ __forceinline__ int gather_tile(
     NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
-    const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int (&mr)[kGT],
-    int (&mc)[kGT]) {
+    const int *acix, const double *scaling, double (&acc)[kGT][kGT + 1], int *inv) {
   constexpr bool F32 = sizeof(CT) == 4;
   int before;
   const int li = front_of(wg_off, nlvl, blockIdx.x, before);
@@ -1392,7 +1402,10 @@ __device__ __forceinline__ int gather_tile(
   }
   const int r0 = I * kGT, c0 = J * kGT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int idx = tid; idx < kGT * kGT; idx += kThreads) acc[idx % kGT][idx / kGT] = 0.0;
+  if (tid < 2 * kGT) {
+#pragma unroll
+    for (int b = 0; b < 3; ++b) inv[2 * kGT * b + tid] = -1;
+  }
   // fully-summed variable list (diagonal tiles own their columns)
   if (I == J) {
     for (int j = c0 + tid; j < min(c0 + kGT, n); j += kThreads) {
@@ -1439,8 +1452,22 @@ __device__ __forceinline__ int gather_tile(
     }
   }
   __syncthreads();
+  // Each wave a 32x32 quadrant in registers: row 16 bi + ri, and with
+  // v_mfma_f64_16x16x4_f64 column 16 bj + kq + 4 rg, with
+  // v_mfma_f32_16x16x4_f32 column 16 bj + 4 kq + rg (the columns' operand is
+  // the first one, so that rows run along the lanes in loads and stores)
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int ri = lane & 15, kq = lane >> 4;
+  auto col = [&](int bj, int rg) { return wc + 16 * bj + (F32 ? 4 * kq + rg : kq + 4 * rg); };
+  const bool below = I != J || wr >= wc;  // not the quadrant above the diagonal
+  double sum[2][2][4];
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) sum[bi][bj][rg] = 0.0;
+  int buf = 0;
   for (int ci = cbeg; ci < cend; ++ci) {
     const NodeDev &c = nodes[child_list[ci]];
     const int cn = c.n, cm = c.m, kb = c.nelim, cldl = c.ldl, cldc = c.ldc;
@@ -1453,56 +1480,59 @@ __device__ __forceinline__ int gather_tile(
     const int kr0 = uni(tab[I]), kr1 = uni(tab[I + 1]);
     const int k0 = uni(tab[J]), k1 = uni(tab[J + 1]);
     if (kr1 <= kr0 || k1 <= k0 || kr1 - 1 < k0) continue;
-    for (int t = tid; t < kr1 - kr0; t += kThreads) mr[t] = cpmap[kr0 + t - kb] - r0;
-    for (int t = tid; t < k1 - k0; t += kThreads) mc[t] = cpmap[k0 + t - kb] - c0;
-    // thread (a, b0): row a of the tile's row range, columns b0, b0+4, ...
-    // (no index division; a wave reads 64 consecutive rows of one column)
-    const int ta = tid & 63, tb = tid >> 6;
-    const int kc0 = max(k0, cn);
-    const int rr0 = max(kr0, cn);
-    const int nrow = kr1 - rr0, ncol = k1 - kc0;
-    const bool contrib = (k1 > kc0 && kr1 > rr0);
-    // C_c, lower part, down its columns: all loads issued before any use
-    constexpr int NU = kGT / (kThreads / 64);
-    CT cv[NU];
-    const bool rowok = contrib && ta < nrow;
-    const int kr = rr0 + ta;
-    // columns b < blim of this thread's row are in the lower part
-    const int blim = rowok ? imin(ncol, kr - kc0 + 1) : 0;
-    {
-      const LoadBuffer<CT> Cb(cC + (size_t)(kc0 - cn) * cldc,
-                              contrib ? (int64_t)kGT * cldc * sizeof(CT) : 0);
-      const unsigned co = (unsigned)(tb * cldc + (kr - cn)) * sizeof(CT);
+    // the child's trailing index at each of the tile's rows (inv[0..63]) and
+    // columns (inv[64..127]), -1 where it has none.  Three copies in turn: one
+    // is read while the one before is cleared and the next filled, so a child
+    // costs one barrier
+    int *iv = inv + 2 * kGT * buf;
+    if (wave == 0 && lane < kr1 - kr0) iv[cpmap[kr0 + lane - kb] - r0] = kr0 + lane;
+    if (wave == 1 && lane < k1 - k0) iv[kGT + cpmap[k0 + lane - kb] - c0] = k0 + lane;
+    __syncthreads();
+    const int last = buf == 0 ? 2 : buf - 1;
+    if (tid < 2 * kGT) inv[2 * kGT * last + tid] = -1;
+    buf = buf == 2 ? 0 : buf + 1;
+    if (!below) continue;
+    int kr[2], kc[2], kcol[2][4];
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int b = tb + u * (kThreads / 64);
-        cv[u] = Cb(b < blim ? co + (unsigned)(u * (kThreads / 64) * cldc) * sizeof(CT)
-                            : kNoLoad);
-      }
+    for (int b = 0; b < 2; ++b) {
+      kr[b] = iv[wr + 16 * b + ri];
+      kc[b] = iv[kGT + wc + 16 * b + ri];
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) kcol[b][rg] = iv[kGT + col(b, rg)];
     }
-    // L21 (L21 D)^T on MFMA: each wave a 32x32 quadrant, operands in the
-    // 16x16x4 fragment layout (lane i+16k holds row i, pivot k) straight
-    // from L21 and the child's L21 D; two register buffers alternate so
-    // the loads of the next 16 pivots are in flight during the MFMAs
+    // failed (delayed) columns of the child: from its panel
+    if (k0 < cn) {
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+          for (int rg = 0; rg < 4; ++rg) {
+            const int k = kcol[bj][rg];
+            if (k >= 0 && k < cn && kr[bi] >= k)
+              sum[bi][bj][rg] += cL[(size_t)k * cldl + kr[bi]];
+          }
+    }
+    // nothing of the contribution block in this quadrant
+    if (!uniform_true(imax(kr[0], kr[1]) >= cn) || !uniform_true(imax(kc[0], kc[1]) >= cn))
+      continue;
+    // L21 (L21 D)^T, operands in the 16x16x4 fragment layout (lane i+16k
+    // holds row i, pivot k) straight from L21 and the child's L21 D; two
+    // register buffers alternate so the loads of the next 8 pivots are in
+    // flight during the MFMAs.  Mixed precision: operands rounded to FP32,
+    // FP32 accumulation
     const int K = kb;
-    const int ra0 = wr + ri, ra1 = ra0 + 16, cb0 = wc + ri, cb1 = cb0 + 16;
-    const bool va0 = ra0 < nrow, va1 = ra1 < nrow, vb0 = cb0 < ncol, vb1 = cb1 < ncol;
-    const unsigned oa0 = va0 ? (unsigned)(kq * cldl + rr0 + ra0) * 8u : kNoLoad;
-    const unsigned oa1 = va1 ? (unsigned)(kq * cldl + rr0 + ra1) * 8u : kNoLoad;
-    const unsigned ob0 = vb0 ? (unsigned)(kq * cldl + kc0 + cb0) * 8u : kNoLoad;
-    const unsigned ob1 = vb1 ? (unsigned)(kq * cldl + kc0 + cb1) * 8u : kNoLoad;
-    // FP64: v_mfma_f64_16x16x4_f64, D[i][j] in lane j + 16 (i % 4), register
-    // i / 4.  Mixed precision: operands rounded to FP32, v_mfma_f32_16x16x4_f32
-    // with FP32 accumulation, D[i][j] in lane j + 16 (i / 4), register i % 4
-    typedef typename std::conditional<F32, float4_t, double4_t>::type acc4_t;
-    acc4_t g[2][2];
+    unsigned oa[2], ob[2];
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < 2; ++bj) g[bi][bj] = (acc4_t){0, 0, 0, 0};
+    for (int b = 0; b < 2; ++b) {
+      oa[b] = kr[b] >= cn ? (unsigned)(kq * cldl + kr[b]) * 8u : kNoLoad;
+      ob[b] = kc[b] >= cn ? (unsigned)(kq * cldl + kc[b]) * 8u : kNoLoad;
+    }
     constexpr int KC = 2;  // k-steps (of 4 pivots) per buffer
-    double xa0[KC], xa1[KC], xb0[KC], xb1[KC], ya0[KC], ya1[KC], yb0[KC], yb1[KC];
-    auto load = [&](int T0, double *A0, double *A1, double *B0, double *B1) {
+    struct Operands {
+      double a[2][KC], b[2][KC];
+    } x, y;
+    auto load = [&](int T0, Operands &o) {
 #pragma unroll
       for (int u = 0; u < KC; ++u) {
         // the length ends with pivot K - 1: a lane whose pivot T + kq is past
@@ -1511,84 +1541,110 @@ __device__ __forceinline__ int gather_tile(
         const int64_t left = (int64_t)(K - T) * cldl * 8;
         const LoadBuffer<double> Lb((const double *)cL + (size_t)T * cldl, left);
         const LoadBuffer<double> Db(cLD + (size_t)T * cldl, left);
-        A0[u] = Lb(oa0);
-        A1[u] = Lb(oa1);
-        B0[u] = Db(ob0);
-        B1[u] = Db(ob1);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          o.a[b][u] = Lb(oa[b]);
+          o.b[b][u] = Db(ob[b]);
+        }
       }
     };
-    auto mfma = [&](int T0, const double *A0, const double *A1, const double *B0,
-                    const double *B1) {
+    load(0, x);
+    // C_c, lower part: all loads issued before any use
+    CT cv[2][2][4];
+    unsigned has = 0;  // bit 8 bi + 4 bj + rg: the block has the entry
+    {
+      const int kc0 = imax(k0, cn);
+      const LoadBuffer<CT> Cb(cC + (size_t)(kc0 - cn) * cldc,
+                              (int64_t)kGT * cldc * sizeof(CT));
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const int k = kcol[bj][rg];
+          const unsigned o = (unsigned)((k - kc0) * cldc - cn) * sizeof(CT);
+#pragma unroll
+          for (int bi = 0; bi < 2; ++bi) {
+            const bool in = k >= cn && kr[bi] >= k;
+            cv[bi][bj][rg] = Cb(in ? o + (unsigned)kr[bi] * sizeof(CT) : kNoLoad);
+            has |= in ? 1u << (8 * bi + 4 * bj + rg) : 0u;
+          }
+        }
+    }
+    if constexpr (F32) load(4 * KC, y);
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) sum[bi][bj][rg] += (double)cv[bi][bj][rg];
+    if constexpr (!F32) load(4 * KC, y);  // (with the FP64 entries: too many registers)
+    typedef typename std::conditional<F32, float4_t, double4_t>::type acc4_t;
+    acc4_t g[2][2];
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj) g[bi][bj] = (acc4_t){0, 0, 0, 0};
+    auto mfma = [&](int T0, const Operands &o) {
 #pragma unroll
       for (int u = 0; u < KC; ++u) {
         if (T0 + 4 * u >= K) break;
-        if constexpr (F32) {
-          const float a0 = (float)A0[u], a1 = (float)A1[u], b0 = (float)B0[u],
-                      b1 = (float)B1[u];
-          g[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, g[0][0], 0, 0, 0);
-          g[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, g[0][1], 0, 0, 0);
-          g[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, g[1][0], 0, 0, 0);
-          g[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, g[1][1], 0, 0, 0);
-        } else {
-          g[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A0[u], B0[u], g[0][0], 0, 0, 0);
-          g[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A0[u], B1[u], g[0][1], 0, 0, 0);
-          g[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A1[u], B0[u], g[1][0], 0, 0, 0);
-          g[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A1[u], B1[u], g[1][1], 0, 0, 0);
-        }
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+          for (int bj = 0; bj < 2; ++bj) {
+            if constexpr (F32)
+              g[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)o.b[bj][u],
+                                                               (float)o.a[bi][u], g[bi][bj],
+                                                               0, 0, 0);
+            else
+              g[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.b[bj][u], o.a[bi][u],
+                                                               g[bi][bj], 0, 0, 0);
+          }
       }
     };
-    // the first two operand buffers go out with the C_c loads, before the
-    // barrier (they depend on the tables only)
-    if (contrib) {
-      load(0, xa0, xa1, xb0, xb1);
-      load(4 * KC, ya0, ya1, yb0, yb1);
+    for (int t0 = 0; t0 < K; t0 += 8 * KC) {
+      if (t0 > 0) load(t0 + 4 * KC, y);
+      mfma(t0, x);
+      if (t0 + 4 * KC >= K) break;
+      load(t0 + 8 * KC, x);
+      mfma(t0 + 4 * KC, y);
     }
-    __syncthreads();  // maps ready
-    // failed (delayed) columns of the child: copy from its panel
-    const int kf1 = min(k1, cn);
-    if (kf1 > k0) {
-      const int nr = kr1 - kr0, ncf = kf1 - k0;
-      if (ta < nr) {
-        const int mra = mr[ta], krr = kr0 + ta;
-        for (int b = tb; b < ncf; b += kThreads / 64) {
-          const int k = k0 + b;
-          if (krr >= k) acc[mra][mc[b]] += cL[(size_t)k * cldl + krr];
-        }
-      }
-    }
-    if (contrib) {
-      if (rowok) {
-        const int mra = mr[rr0 - kr0 + ta];
 #pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const int b = tb + u * (kThreads / 64);
-          if (b < blim) acc[mra][mc[kc0 - k0 + b]] += (double)cv[u];
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const double v = sum[bi][bj][rg] - (double)g[bi][bj][rg];
+          sum[bi][bj][rg] = (has >> (8 * bi + 4 * bj + rg) & 1) ? v : sum[bi][bj][rg];
         }
-      }
-      for (int t0 = 0; t0 < K; t0 += 8 * KC) {
-        if (t0 > 0) load(t0 + 4 * KC, ya0, ya1, yb0, yb1);
-        mfma(t0, xa0, xa1, xb0, xb1);
-        if (t0 + 4 * KC >= K) break;
-        load(t0 + 8 * KC, xa0, xa1, xb0, xb1);
-        mfma(t0 + 4 * KC, ya0, ya1, yb0, yb1);
-      }
-      __syncthreads();  // the C_c pass has finished with acc
+  }
+  // a tile without A entries goes to the front from the registers
+  if (PART != 1 && ae1 <= ae0) {
+    if (below) {
 #pragma unroll
       for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg) {
-            const int i = wr + bi * 16 + (F32 ? 4 * kq + rg : kq + 4 * rg);
-            const int j = wc + bj * 16 + ri;
-            if (i < nrow && j < ncol) {
-              const int krr = rr0 + i, k = kc0 + j;
-              if (krr >= k) acc[mr[krr - kr0]][mc[k - k0]] -= (double)g[bi][bj][rg];
+            const int gr = r0 + wr + 16 * bi + ri, gc = c0 + col(bj, rg);
+            if (gr < m && gr >= gc) {
+              if (gc < n) PL[(size_t)gc * pldl + gr] = sum[bi][bj][rg];
+              else PC[(size_t)(gc - n) * pldc + (gr - n)] = (CT)sum[bi][bj][rg];
             }
           }
     }
-    __syncthreads();
+    return (I == 0 && J == 0) ? s : -1;
   }
+#pragma unroll
+  for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+        acc[wr + 16 * bi + ri][col(bj, rg)] = sum[bi][bj][rg];
+  __syncthreads();
   // A entries
 #pragma unroll
   for (int u = 0; u < kAE; ++u) {
@@ -1621,14 +1677,14 @@ __device__ __forceinline__ int gather_tile(
 }
 
 template <int PART, typename CT>
-__global__ __launch_bounds__(kThreads, 4) void k_gather(
+__global__ __launch_bounds__(kThreads, sizeof(CT) == 4 ? 4 : 3) void k_gather(
     NodeDev *nodes, int s0, const int *wg_off, int nlvl,
     const int *child_list, const double *aval, const int64_t *asrc, const int *arow,
     const int *acix, const double *scaling) {
   __shared__ double acc[kGT][kGT + 1];
-  __shared__ int mr[kGT], mc[kGT];
+  __shared__ int inv[kGatherInv];
   gather_tile<PART, CT>(nodes, s0, wg_off, nlvl, child_list, aval, asrc, arow, acix,
-                        scaling, acc, mr, mc);
+                        scaling, acc, inv);
 }
 
 
