@@ -56,6 +56,9 @@ struct NodeDev {
   int nelim_app;
   int flag;         // 0 ok, -5 singular (action false)
   int nzero;
+  // an update whose tiles beyond the first tile column run beside the next
+  // pivot block: its first column, and its step + 1
+  int ahead_p, ahead_step;
   int lp[kBlk];
   unsigned long long fail;  // columns of the step's block with an |l| above 1/u
 };

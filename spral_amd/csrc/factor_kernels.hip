@@ -17,6 +17,8 @@
 //  k_update     restore failed columns and apply the accepted pivots to the
 //               trailing panel columns with v_mfma_f64_16x16x4_f64 on 64x64
 //               tiles (the contribution block is updated lazily by k_gather).
+//  k_update_diag  on large fronts, all but the first tile column of that,
+//               beside the next step's pivot blocks.
 //  k_swap       move failed columns behind the unprocessed candidates.
 //  k_tail       end of a level, one workgroup per front: APP result,
 //               threshold partial pivoting on the failed columns
@@ -323,8 +325,8 @@ struct GatherArgs {  // the level's gather inputs (a pivot launch that assembles
 // twice as many workgroups on a CU.
 // C32 (FIRST only): the children's contribution blocks are FP32
 template <int NW, bool FIRST, bool C32>
-__global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, int s0,
-                                                  int step, FactorParams fp, GatherArgs ga) {
+__device__ __forceinline__ void diag_front(NodeDev *nodes, int s0, int step, FactorParams fp,
+                                           GatherArgs ga) {
   constexpr int R = kBlk / NW;
   static_assert(NW == kDiagWaves && R == kDiagCols, "a row of lanes holds L of a wave's columns");
   __shared__ double t[kBlk][kBlk + 1];  // load staging, then L by step: t[k][row]
@@ -637,6 +639,11 @@ __global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, int s0,
   const int pv = (tid < w) ? N.perm[p + lp[tid]] : 0;
   __syncthreads();
   if (tid < w) N.perm[p + tid] = pv;
+}
+template <int NW, bool FIRST, bool C32>
+__global__ __launch_bounds__(64 * NW) void k_diag(NodeDev *nodes, int s0,
+                                                  int step, FactorParams fp, GatherArgs ga) {
+  diag_front<NW, FIRST, C32>(nodes, s0, step, fp, ga);
 }
 
 // ---------------------------------------------------------------------------
@@ -1121,10 +1128,27 @@ __device__ __forceinline__ void update_tiles(gdouble *NL, int ldl, gcdouble *X, 
   }
 }
 
+// Workgroup `local` of `count` on tiles [first, first + ntiles): a run of
+// consecutive tiles each; workgroups go to the eight XCDs in turn, and the runs
+// of one XCD's workgroups are neighbours, so that its L2 holds the operands of
+// few tile columns.
+__device__ __forceinline__ void update_run(gdouble *NL, int ldl, gcdouble *X, int ldx, int p,
+                                           int m, int n, int TI, int TJ, int first, int ntiles,
+                                           int local, int count) {
+  const int used = imin(count, ntiles);
+  if (local >= used) return;
+  const int c8 = used >> 3;
+  const int run = (local < 8 * c8) ? (local & 7) * c8 + (local >> 3) : local;
+  const int tb = (int)((int64_t)run * ntiles / used);
+  const int te = (int)((int64_t)(run + 1) * ntiles / used);
+  update_tiles(NL, ldl, X, ldx, p, m, n, TI, TJ, first + tb, first + te);
+}
+
 __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
                                                            int s0,
                                                            const int *wg_off, int nlvl,
-                                                           int step, FactorParams fp) {
+                                                           int step, int ahead,
+                                                           FactorParams fp) {
   __shared__ double ce1[kBlk], ce2[kBlk];
   __shared__ int ctwo[kBlk];
   int before;
@@ -1146,19 +1170,13 @@ __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
   const int TI = (m - t0 + kTile - 1) / kTile, TJ = (cend - t0 + kTile - 1) / kTile;
   const int ntiles = TJ * TI - TJ * (TJ - 1) / 2;
   if (np == kBlk) {
-    gdouble *NL = (gdouble *)nL;
-    gcdouble *X = (gcdouble *)nX;
-    const int ldl = nl, ldx = nldbak;
-    // a run of consecutive tiles each; workgroups go to the eight XCDs in
-    // turn, and the runs of one XCD's workgroups are neighbours, so that its
-    // L2 holds the operands of few tile columns
-    const int used = imin(count, ntiles);
-    if (local >= used) return;
-    const int c8 = used >> 3;
-    const int run = (local < 8 * c8) ? (local & 7) * c8 + (local >> 3) : local;
-    const int tb = (int)((int64_t)run * ntiles / used);
-    const int te = (int)((int64_t)(run + 1) * ntiles / used);
-    update_tiles(NL, ldl, X, ldx, p, m, cend, TI, TJ, tb, te);
+    // ahead: the first tile column, the rest beside the next pivot block
+    if (ahead && local == 0 && tid == 0) {
+      N.ahead_p = p;
+      N.ahead_step = step + 1;
+    }
+    update_run((gdouble *)nL, nl, (gcdouble *)nX, nldbak, p, m, cend, TI, TJ, 0,
+               ahead ? TI : ntiles, local, count);
     return;
   }
   {
@@ -1270,6 +1288,37 @@ __global__ __launch_bounds__(kThreads, 2) void k_update_panel(NodeDev *nodes,
           }
         }
   }
+}
+
+// The next step's pivot blocks (a workgroup per front, the first ones) beside
+// what k_update_panel left of this step's update: when a front's whole block
+// passed, the tiles beyond the first tile column, which the pivot blocks do
+// not touch.  A pivot block is a chain on one CU (56 us in a 64^3
+// factorization) that needs the first tile column only, and the rest of the
+// update takes up to 90 us of the other CUs; one after the other they bounded
+// every step of a large front.  The launch takes enough LDS for one workgroup
+// a CU, `share` of them a front in one round: an update workgroup on a pivot
+// block's CU shares its FP64 units (72 us a launch against 63).  64^3 refactor
+// + solve 34.9 -> 32.7 ms.  What is left of the update is read from ahead_p and
+// ahead_step, as the pivot block moves p on; the apply, which overwrites L21 D
+// and moves rows of this step's L, comes after this launch.
+__global__ __launch_bounds__(kThreads, 1) void k_update_diag(NodeDev *nodes, int s0, int nlvl,
+                                                          int share, int step,
+                                                          FactorParams fp) {
+  if (blockIdx.x < (unsigned)nlvl) {
+    diag_front<kDiagWaves, false, false>(nodes, s0, step + 1, fp, GatherArgs{});
+    return;
+  }
+  const int b = blockIdx.x - nlvl, local = b / nlvl;
+  NodeDev &N = nodes[s0 + (b - local * nlvl)];
+  const int p = N.ahead_p, tag = N.ahead_step, m = N.m, n = N.n, ldl = N.ldl, ldx = N.ldbak;
+  double *const nL = N.L, *const nX = N.X;
+  loaded(p, tag, m, n, ldl, ldx, nL, nX);
+  if (tag != step + 1) return;
+  const int t0 = p + kBlk;
+  const int TI = (m - t0 + kTile - 1) / kTile, TJ = (n - t0 + kTile - 1) / kTile;
+  update_run((gdouble *)nL, ldl, (gcdouble *)nX, ldx, p, m, n, TI, TJ, TI,
+             TJ * TI - TJ * (TJ - 1) / 2 - TI, local, share);
 }
 
 // D (not its inverse) per pivot for the lazy contribution update:
@@ -2602,14 +2651,22 @@ void launch_apply(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                        nlvl, step, fp);
 }
 void launch_update(hipStream_t st, int nwg, NodeDev *nodes, int s0,
-                   const int *wg_off, int nlvl, int step, int mode, FactorParams fp) {
+                   const int *wg_off, int nlvl, int step, int mode, int ahead,
+                   FactorParams fp) {
   if (nwg <= 0) return;
   if (mode == 0)
     hipLaunchKernelGGL(k_update_panel, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
-                       nlvl, step, fp);
+                       nlvl, step, ahead, fp);
   else
     hipLaunchKernelGGL(k_update, dim3(nwg), dim3(kThreads), 0, st, nodes, s0, wg_off,
                        nlvl, step, mode, fp);
+}
+void launch_update_diag(hipStream_t st, int share, NodeDev *nodes, int s0, int nlvl, int step,
+                        FactorParams fp) {
+  // LDS past half a CU's: one workgroup a CU
+  constexpr unsigned kAlone = 12 << 10;
+  hipLaunchKernelGGL(k_update_diag, dim3(nlvl * (1 + share)), dim3(kThreads), kAlone, st,
+                     nodes, s0, nlvl, share, step, fp);
 }
 void launch_swap(hipStream_t st, int nwg, NodeDev *nodes, int s0,
                  const int *wg_off, int nlvl, int step) {

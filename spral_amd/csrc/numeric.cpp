@@ -39,8 +39,9 @@ void launch_maptab(hipStream_t, int, NodeDev *, int, const int *);
 void launch_diag(hipStream_t, int, NodeDev *, int, int, FactorParams);
 void launch_apply(hipStream_t, int, NodeDev *, int, const int *, int, int,
                   FactorParams);
-void launch_update(hipStream_t, int, NodeDev *, int, const int *, int, int, int,
+void launch_update(hipStream_t, int, NodeDev *, int, const int *, int, int, int, int,
                    FactorParams);
+void launch_update_diag(hipStream_t, int, NodeDev *, int, int, int, FactorParams);
 void launch_swap(hipStream_t, int, NodeDev *, int, const int *, int, int);
 void launch_tail(hipStream_t, int, NodeDev *, int, FactorParams, int *);
 void launch_stats(hipStream_t, const NodeDev *, int, int *, const FactorParams &);
@@ -256,6 +257,9 @@ struct Plan {
     int maxsteps = 0;
     size_t tab_off = 0;
     std::vector<int> cap;                   // capacity workgroups per table
+    std::vector<int> ahead;                 // per step: 0, or the next pivot block runs
+                                            // beside the update, which has so many
+                                            // workgroups a front (k_update_diag)
   };
   std::vector<Level> lv;
   int *d_tabs = nullptr;
@@ -807,6 +811,23 @@ static void plan_build(Numeric &N, int pivot_tpp, double multiplier) {
       for (int li = 0; li < nl; ++li)
         lv.cap[t] += level_table_count(t, lv.maxsteps, mc[li], nc[li], sc[li],
                                        P.tmpl[s0 + li].is_root);
+    // Beside the next pivot block from kAheadTiles tiles on: below that the
+    // update takes 8 to 20 us, as long as its first tile column by itself.
+    // The fronts share the other CUs evenly, so not where the largest front's
+    // share would take much longer than a pivot block (2 us a tile).
+    constexpr int kCus = 256, kAheadTiles = 1024, kAheadRun = 40;
+    lv.ahead.assign(std::max(lv.maxsteps, 1), 0);
+    const int share = (kCus - nl) / nl;
+    for (int stp = 0; stp + 1 < lv.maxsteps && share > 0; ++stp) {
+      int64_t tiles = 0, most = 0;
+      for (int li = 0; li < nl; ++li) {
+        const int64_t TI = cdiv(std::max(mc[li] - (stp + 1) * kBlk, 0), kBlk);
+        const int64_t TJ = cdiv(std::max(nc[li] - (stp + 1) * kBlk, 0), kBlk);
+        tiles += TJ * TI - TJ * (TJ - 1) / 2;
+        most = std::max(most, TJ * TI - TJ * (TJ - 1) / 2 - TI);
+      }
+      if (tiles > kAheadTiles && most <= (int64_t)kAheadRun * share) lv.ahead[stp] = share;
+    }
     lv.tab_off = tab_total;
     tab_total += (size_t)ntab * (nl + 1);
     // this level's fronts have consumed their children's blocks
@@ -908,7 +929,7 @@ static bool factor_static(Numeric &N, const FactorParams &fp, const spral_ssids_
       joined = true;
     };
     for (int stp = 0; stp < ms; ++stp) {
-      if (stp > 0) launch_diag(st, nl, N.d_nodes, s0, stp, fp);
+      if (stp > 0 && !lv.ahead[stp - 1]) launch_diag(st, nl, N.d_nodes, s0, stp, fp);
       // step 0's apply reads the whole first tile column
       if (stp == 0) HIPCHK(hipStreamWaitEvent(st, N.ev_first, 0));
       launch_apply(st, lv.cap[1 + stp], N.d_nodes, s0, toff(1 + stp), nl, stp, fp);
@@ -916,15 +937,18 @@ static bool factor_static(Numeric &N, const FactorParams &fp, const spral_ssids_
       // column too; with more steps it reaches the later columns
       if (ms > 1) join();
       launch_update(st, lv.cap[ms + 2 + stp], N.d_nodes, s0, toff(ms + 2 + stp), nl, stp,
-                    0, fp);
+                    0, lv.ahead[stp] > 0, fp);
       // (the last step leaves no unprocessed candidate to swap with)
       if (stp + 1 < ms)
         launch_swap(st, lv.cap[ms + 1], N.d_nodes, s0, toff(ms + 1), nl, stp);
+      if (lv.ahead[stp])
+        launch_update_diag(st, lv.ahead[stp], N.d_nodes, s0, nl, stp, fp);
     }
     join();
     launch_tail(st, nl, N.d_nodes, s0, fp, N.d_scratch_n);
     if (lv.cap[2 * ms + 2] > 0)
-      launch_update(st, lv.cap[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1, fp);
+      launch_update(st, lv.cap[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1,
+                    0, fp);
   }
   launch_pack_nodes(st, N.d_nodes, nn, P.d_pack);
   };
@@ -1075,14 +1099,15 @@ static void factor_dynamic(Numeric &N, const FactorParams &fp,
     for (int stp = 0; stp < ms; ++stp) {
       launch_diag(st, nl, N.d_nodes, s0, stp, fp);
       launch_apply(st, tot[1 + stp], N.d_nodes, s0, toff(1 + stp), nl, stp, fp);
-      launch_update(st, tot[ms + 2 + stp], N.d_nodes, s0, toff(ms + 2 + stp), nl, stp, 0,
+      launch_update(st, tot[ms + 2 + stp], N.d_nodes, s0, toff(ms + 2 + stp), nl, stp, 0, 0,
                     fp);
       if (stp + 1 < ms)
         launch_swap(st, tot[ms + 1], N.d_nodes, s0, toff(ms + 1), nl, stp);
     }
     launch_tail(st, nl, N.d_nodes, s0, fp, N.d_scratch_n);
     if (tot[2 * ms + 2] > 0)
-      launch_update(st, tot[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1, fp);
+      launch_update(st, tot[2 * ms + 2], N.d_nodes, s0, toff(2 * ms + 2), nl, 0, 1,
+                    0, fp);
     HIPCHK(hipGetLastError());
     // read back the level's results (nelim, flag)
     std::vector<NodeDev> back(nl);

@@ -90,3 +90,32 @@ def test_grid_groups(lib, nrhs):
         y = gpu_solve(ak, fk, opts, y, job=ssids.SSIDS_SOLVE_JOB_DIAG_BWD)
         assert np.allclose(y, x, rtol=1e-12, atol=1e-12)
         ssids.ssids_free(ak, fk)
+
+
+@pytest.mark.parametrize("n,weak", [(2944, ()), (2945, (0, 192)), (3001, (0, 1, 2, 704))])
+def test_update_beside_pivot_block(lib, monkeypatch, n, weak):
+    """Trailing updates split around the next pivot block (over 1,024 tiles at
+    the first steps) give the level-by-level path's bits, with whole blocks and
+    with blocks whose columns fail (a diagonal block of 1e-6 entries)."""
+    print(f"update beside pivot block n={n} weak={weak}", flush=True)
+    rng = np.random.default_rng(n)
+    a = rng.uniform(-1.0, 1.0, (n, n))
+    a = np.tril(a) + np.tril(a, -1).T + np.diag(rng.choice([-80.0, 80.0], n))
+    for k in weak:
+        a[k:k + 64, k:k + 64] *= 1e-6
+    m = dense_lower(a)
+    ak, _ = analyse(m, use_gpu=True)
+    _, b = rhs(m, 1, 8)
+    got = []
+    for env in ("0", "1"):
+        monkeypatch.setenv("SPRAL_SSIDS_HIP_NO_PLAN", env)
+        fk, inf = ssids.ssids_factor(False, m.val, ak, ssids.SSIDSOptions())
+        assert inf.flag >= 0
+        x = b.copy()
+        assert ssids.ssids_solve(x, ak, fk, ssids.SSIDSOptions()).flag >= 0
+        got.append((x, inf.num_neg, inf.num_two, inf.not_first_pass, inf.not_second_pass))
+        ssids.ssids_free(None, fk)
+    assert np.array_equal(got[0][0], got[1][0]) and got[0][1:] == got[1][1:]
+    assert matrices.bwd_error(m.full, got[0][0], b).max() <= 1e-12
+    assert (got[0][3] > 0) == bool(weak)
+    ssids.ssids_free(ak)
