@@ -1383,7 +1383,8 @@ __global__ __launch_bounds__(kThreads) void k_maptab(NodeDev *nodes, int s0,
 // tiles: of every 1,024 (what runs at once) an XCD takes 128 in sequence, in
 // strips of eight tile columns traversed by rows.  The 128 tiles read some 16
 // + 8 rows of 64 of the children's L21 and L21 D; down the columns and across
-// the XCDs it was up to T + 16.
+// the XCDs it was up to T + 16.  64^3: 1,396 -> 749 MB read a launch; 32^3
+// 27-point KKT, mixed: 78.3 -> 74.4 ms.
 constexpr int kXcd = 8, kXcdRun = 128, kStrip = 8;
 __device__ inline void gather_place(int local, int count, int T, int jfirst, int &I, int &J) {
   const int base = local & ~(kXcd * kXcdRun - 1), l = local - base;
